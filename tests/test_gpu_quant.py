@@ -72,6 +72,27 @@ def test_quant_fp16_fp32_match_eager(dev, dtype):
     assert torch.equal(s.cpu(), s_ref)
 
 
+# Row widths around the register kernel's edges: one 16-byte chunk, a partly filled wave, a row per
+# wave (3072, 4104) and per workgroup (wide rows and few rows), and widths whose chunks are not aligned.
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("m,k", [(1, 8), (3, 520), (5, 2052), (4097, 72), (4100, 3072), (4099, 4104), (7, 14336),
+                                 (4098, 8200), (2, 65536), (9, 1001)])
+def test_quant_row_widths_match_eager(dev, dtype, m, k):
+    print(f"quant {dtype} m={m} k={k}", flush=True)
+    x = (torch.randn(m, k, generator=gen(m * 7 + k)) * 3).to(dtype)
+    x[0] = 0
+    if m > 2:
+        x[1, k // 2] = float("inf")
+        x[2, k - 1] = float("nan")
+    if m > 4:
+        x[3] = x[3] * 1e-6  # float16: subnormal values, a scale that rounds to zero or below normal
+        x[4] = x[4] * 1e3
+    q, s = _mx().quantize_int8_rowwise(x.to(dev))
+    q_ref, s_ref = eager_torch.quantize_int8_rowwise(x)
+    assert torch.equal(q.cpu(), q_ref)
+    assert torch.equal(s.cpu().nan_to_num(-1.0), s_ref.nan_to_num(-1.0))
+
+
 def test_quant_row_slices_are_independent(dev):
     """Quantizing a row range equals the same rows of the full result (per-token scales)."""
     x = activations(300, 3072, seed=11).to(dev)
