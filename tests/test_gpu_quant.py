@@ -299,6 +299,26 @@ def test_adaln_modulation_groups(dev, m, rows_per_group, d):
         assert torch.equal(y[rows], yg)
 
 
+# Scale and shift rows over groups of their own: runs of whole rows (equal, nested either way, one
+# of them shared by all), groups that do not nest (read per row), more than 1024 runs of fewer and
+# of at least 4 rows, and rows left over in the last run's wave slots.
+@pytest.mark.parametrize("m,scale_rows,shift_rows,d", [(35, 7, 7, 5120), (36, 12, 4, 520), (36, 4, 12, 1024),
+                                                       (36, 36, 6, 3072), (36, 6, 36, 3072), (36, 9, 6, 512),
+                                                       (2052, 2, 2, 512), (4104, 4, 4, 512)])
+def test_adaln_quant_runs(dev, m, scale_rows, shift_rows, d):
+    x = activations(m, d, 78)
+    sc = (torch.randn(m // scale_rows, d, generator=gen(1)) * 0.1).to(torch.bfloat16)
+    sh = (torch.randn(m // shift_rows, d, generator=gen(2)) * 0.1).to(torch.bfloat16)
+    got = _mx().adaln_quantize_int8(x.to(dev), sc.to(dev), sh.to(dev), return_modulated=True)
+    step = min(scale_rows, shift_rows) if max(scale_rows, shift_rows) % min(scale_rows, shift_rows) == 0 else 3
+    for a in range(0, m, step * max(1, m // step // 40)):  # one modulation row for these rows
+        b = a + step
+        want = _mx().adaln_quantize_int8(x[a:b].to(dev), sc[a // scale_rows].to(dev), sh[a // shift_rows].to(dev),
+                                         return_modulated=True)
+        for g, w in zip(got, want):
+            assert torch.equal(g[a:b], w), (a, b)
+
+
 def _nan_inf_rows(m, k, dtype, seed):
     """Rows with a NaN, with +-inf, with both, and plain rows (torch's amax propagates NaN)."""
     x = activations(m, k, seed).to(dtype)

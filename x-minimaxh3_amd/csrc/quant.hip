@@ -473,6 +473,13 @@ MXQ_DEVICE void adaln_row(const uint16_t* __restrict__ x, const v4u* scv, const 
 // t = bf16(1 + scale) once and keeps t and shift in LDS; otherwise each row reads its modulation
 // from global memory.
 constexpr int kAdalnRows = 16;
+// Runs (rows that share one modulation row) shorter than kAdalnMinRun rows go to adaln_uniform_rows
+// only while they number at most kAdalnFewRuns: each of its workgroups stages cols * 8 bytes of
+// modulation for its run. Measured against the per-row form (us, 5120 columns, quantizer included):
+// 32760 rows in 2 runs 102 against 190, runs of 64 / 16 / 4 rows 107 / 112 / 182 against 187 / 187 /
+// 235, of 2 and 1 rows 294 and 699 against 237 and 271 (3072 columns: 161 and 275 against 289 and 292);
+// 960 rows in runs of 1 row 15.0 against 38.5.
+constexpr int64_t kAdalnMinRun = 4, kAdalnFewRuns = 1024;
 constexpr int kAdalnMaxCols = 8192;
 
 template <int NCH, bool kQuant>
@@ -514,8 +521,8 @@ __global__ __launch_bounds__(kQuantBlock) void adaln_rows_reg(
   }
 }
 
-// adaLN with one modulation row for every row (the common case: one sample per launch). One wave
-// per row, rows taken grid-stride by the launch's waves; each wave loads its next row into a
+// adaLN with one modulation row for each run of `run` consecutive rows (one run per sample:
+// blockIdx.y). One wave per row, a run's rows taken grid-stride by its workgroups' waves; each wave loads its next row into a
 // second register buffer before it processes the current one, so a row's HBM latency overlaps
 // the previous row's arithmetic. t = bf16(1 + scale) and shift are staged once per workgroup in
 // LDS as fp32 (cols * 8 bytes of dynamic LDS). The statistics and the modulation are the same
@@ -531,8 +538,11 @@ MXQ_DEVICE void unpack_fresh(uint32_t w, float& lo, float& hi) {
 template <int NCH, bool kQuant, bool kExact>
 __global__ __launch_bounds__(kQuantBlock) __attribute__((amdgpu_waves_per_eu(kExact && NCH <= 10 ? 3 : 2))) void adaln_uniform_rows(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ scale, const uint16_t* __restrict__ shift,
-    float eps, int8_t* __restrict__ q, float* __restrict__ scales, uint16_t* __restrict__ y_out, int64_t rows,
-    int cols) {
+    int64_t scale_group, int64_t shift_group, int64_t run, float eps, int8_t* __restrict__ q,
+    float* __restrict__ scales, uint16_t* __restrict__ y_out, int64_t all_rows, int cols) {
+  const int64_t first = (int64_t)blockIdx.y * run, rows = min(first + run, all_rows);
+  scale += first / scale_group * cols;
+  shift += first / shift_group * cols;
   extern __shared__ __attribute__((aligned(16))) float s_mod[];
   float* s_t = s_mod;
   float* s_sh = s_mod + cols;
@@ -544,7 +554,7 @@ __global__ __launch_bounds__(kQuantBlock) __attribute__((amdgpu_waves_per_eu(kEx
   const int lane = threadIdx.x % kWave;
   const int nchunk = kExact ? NCH * kWave : cols / 8;  // kExact: cols == NCH * 512
   const int64_t stride = (int64_t)gridDim.x * (kQuantBlock / kWave);
-  int64_t row = (int64_t)blockIdx.x * (kQuantBlock / kWave) + threadIdx.x / kWave;
+  int64_t row = first + (int64_t)blockIdx.x * (kQuantBlock / kWave) + threadIdx.x / kWave;
 
   // Loads are unconditional (a chunk past the row end re-reads the row's last chunk and is masked
   // out of the statistics, the absmax and the stores): a load inside a branch made the compiler
@@ -939,23 +949,32 @@ static int adaln_launch(const void* x, const void* scale, const void* shift, int
   const int64_t need = (cols / 8 + kWave - 1) / kWave;
   const int uch = need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : need <= 6 ? 6 : need <= 8 ? 8 : need <= 10 ? 10
                 : need <= 11 ? 11 : need <= 12 ? 12 : need <= 14 ? 14 : 16;
-  if (scale_group >= rows && shift_group >= rows && cols <= kAdalnMaxCols && (cols == uch * 512 || uch <= 12)) {
-    // one modulation row: the two-buffer kernel (widths whose register budget it fits)
+  // Rows per run that share one scale row and one shift row, where both groups start together.
+  int64_t run = 0;
+  if (scale_group >= rows && shift_group >= rows)
+    run = rows;
+  else if (scale_group >= rows || (scale_group >= shift_group && scale_group % shift_group == 0))
+    run = shift_group;
+  else if (shift_group >= rows || shift_group % scale_group == 0)
+    run = scale_group;
+  const int64_t runs = run ? (rows + run - 1) / run : 0;
+  if (run && (runs <= kAdalnFewRuns || (run >= kAdalnMinRun && runs <= 65535)) && cols <= kAdalnMaxCols && (cols == uch * 512 || uch <= 12)) {
+    // few modulation rows: the two-buffer kernel (widths whose register budget it fits)
     // Every workgroup takes an equal share of the rows, so the grid is what fits on the device at
     // once: a larger one left its last workgroups to start after the first had finished.
     const size_t lds = (size_t)cols * 2 * sizeof(float);
-    const int64_t wg = (rows + kRowsPerBlock - 1) / kRowsPerBlock;
-#define MXQ_ADALN_UNIFORM_K(N_, E_)                                                                              \
-  (quant ? (void)(adaln_uniform_rows<N_, true, E_><<<mxq_resident_grid(adaln_uniform_rows<N_, true, E_>,          \
-                                                                       kQuantBlock, lds, wg),                    \
-                                                     kQuantBlock, lds, st>>>(                                    \
-               (const uint16_t*)x, (const uint16_t*)scale, (const uint16_t*)shift, eps, q, scales,              \
-               (uint16_t*)y_out, rows, (int)cols))                                                               \
-         : (void)(adaln_uniform_rows<N_, false, E_><<<mxq_resident_grid(adaln_uniform_rows<N_, false, E_>,        \
-                                                                        kQuantBlock, lds, wg),                   \
-                                                      kQuantBlock, lds, st>>>(                                   \
-               (const uint16_t*)x, (const uint16_t*)scale, (const uint16_t*)shift, eps, nullptr, nullptr,        \
-               (uint16_t*)y_out, rows, (int)cols)))
+    const int64_t wg = (run + kRowsPerBlock - 1) / kRowsPerBlock;
+    auto grid = [&](auto kernel) {
+      const int64_t resident = mxq_resident_grid(kernel, kQuantBlock, lds, INT32_MAX);
+      return dim3((unsigned)std::min(wg, std::max<int64_t>(resident / runs, 1)), (unsigned)runs);
+    };
+#define MXQ_ADALN_UNIFORM_K(N_, E_)                                                                             \
+  (quant ? (void)(adaln_uniform_rows<N_, true, E_><<<grid(adaln_uniform_rows<N_, true, E_>), kQuantBlock, lds, st>>>( \
+               (const uint16_t*)x, (const uint16_t*)scale, (const uint16_t*)shift, scale_group, shift_group, run,    \
+               eps, q, scales, (uint16_t*)y_out, rows, (int)cols))                                              \
+         : (void)(adaln_uniform_rows<N_, false, E_><<<grid(adaln_uniform_rows<N_, false, E_>), kQuantBlock, lds, st>>>( \
+               (const uint16_t*)x, (const uint16_t*)scale, (const uint16_t*)shift, scale_group, shift_group, run,    \
+               eps, nullptr, nullptr, (uint16_t*)y_out, rows, (int)cols)))
 #define MXQ_ADALN_UNIFORM(N_) \
   (cols == (N_) * 512 ? MXQ_ADALN_UNIFORM_K(N_, true) : MXQ_ADALN_UNIFORM_K(N_, false))
     switch (uch) {
