@@ -59,20 +59,23 @@ constexpr int kGemmThreads = 256;                       // 4 waves as 2 x 2
 // kTN = 96 (deep ring only): 128 x 96 tiles, the four waves stacked as 32-row strips of 1 x 3
 // blocks, for problems that fill more CUs that way (1024 x 3072: 256 tiles instead of 192 of 128).
 // A B chunk is then 12 KB in a 16 KB slot, and the ring carries 28 KB per stage instead of 32.
-template <int kT, bool kDeep = false, bool kPP = false, int kTN = kT>
+// kTM = 64, 32: 64 or 32 rows of the same deep ring, the four waves side by side along the columns, for
+// the K slices of problems of that few rows (split_plan).
+template <int kT, bool kDeep = false, bool kPP = false, int kTN = kT, int kTM = kT>
 struct TileCfg {
   static_assert(kT == 128 || !kDeep, "the deep ring exists for 128-tiles only");
   static_assert(kT == 256 || !kPP, "the ping-pong schedule exists for 256-tiles only");
   static_assert(kTN == kT || (kDeep && kTN == 96), "128 x 96 tiles run the deep ring only");
+  static_assert(kTM == kT || (kDeep && kTN == kT && (kTM == 64 || kTM == 32)), "few-row tiles run the deep ring only");
   static constexpr bool kPingPong = kPP;
   static constexpr int kWaves = kPP ? 8 : 4;                    // two per SIMD with kPP
   static constexpr int kThreads = kWaves * 64;
-  static constexpr int kBM = kT, kBN = kTN;
-  static constexpr int kWavesN = kPP ? 4 : (kTN == kT ? 2 : 1);  // waves across the tile's columns
-  static constexpr int kWaveM = kPP ? kT / 2 : kT / (kWaves / kWavesN), kWaveN = kTN / kWavesN;
+  static constexpr int kBM = kTM, kBN = kTN;
+  static constexpr int kWavesN = kPP || kTM < kT ? 4 : (kTN == kT ? 2 : 1);  // waves across the tile's columns
+  static constexpr int kWaveM = kPP ? kT / 2 : kTM / (kWaves / kWavesN), kWaveN = kTN / kWavesN;
   static constexpr int kBI = kWaveM / 32, kBJ = kWaveN / 32;
   static constexpr int kSlotBytes = kT * kBK;                  // one operand chunk of a stage (slot size)
-  static constexpr int kLoads = kSlotBytes / 1024 / kWaves;     // direct-to-LDS loads per wave per A slot
+  static constexpr int kLoads = kTM * kBK / 1024 / kWaves;      // direct-to-LDS loads per wave per A slot
   static constexpr int kLoadsB = kTN * kBK / 1024 / kWaves;     // ... per B slot
   static constexpr int kAhead = kDeep ? 4 : 2;                  // stages requested ahead of the MFMAs
   static constexpr int kSlots = 2 * kAhead + 1;                 // LDS ring of operand chunks
@@ -95,7 +98,7 @@ struct TileCfg {
 // own (plan_gemm).
 constexpr int kGroupM = 2, kGroupMPingPong = 4;
 
-enum { kEpiI32 = 0, kEpiDequant = 1, kEpiGelu = 2, kEpiGatedRes = 3, kEpiSwiGLU = 4 };
+enum { kEpiI32 = 0, kEpiDequant = 1, kEpiGelu = 2, kEpiGatedRes = 3, kEpiSwiGLU = 4, kEpiSplit = 5 };
 // Table epilogues as plan_gemm sees them: GELU keeps the whole 128 KB table in LDS (four-wave
 // 256-tiles), SwiGLU the 8 KB compact SiLU table (ping-pong 256-tiles).
 enum { kTableGelu = 1, kTableSwiGLU = 2 };
@@ -127,6 +130,10 @@ struct GemmArgs {
   // Ping-pong kernel only: wg_per_xcd workgroups per XCD loop over the tiles, claiming them from
   // the counters (pp_tiles); n_claim is then the grid.
   int persistent;
+  // Split K (kEpiSplit): `splits` slices of slice_k K-bytes each (a multiple of kBK), slice s writing its int32 sums
+  // at d + s * slice_stride.
+  int splits;
+  int64_t slice_k, slice_stride;
 };
 
 // LDS operand layout: a tile row is 128 bytes = eight 16-byte chunks; chunk c of row r sits at
@@ -271,18 +278,21 @@ MXQ_DEVICE void mma_step(const v4i fa[C::kBI], const v4i fb[C::kBJ], v16i acc[C:
 }
 
 // The MFMAs of one K-step with kCount direct-to-LDS loads (loads kFirst .. of one operand slot)
-// interleaved, one after each of the first kCount MFMAs (kCount <= kBI * kBJ). Spread this way,
+// interleaved, one after each of the first kCount MFMAs. Spread this way,
 // a load that waits for room in the memory pipeline holds up the wave while its MFMAs still
 // run, rather than after the last of them.
 template <class C, bool kB, int kFirst, int kCount, bool kCheck>
 MXQ_DEVICE void mma_step_dma(const v4i fa[C::kBI], const v4i fb[C::kBJ], v16i acc[C::kBI][C::kBJ],
                              const Loader<C::kLoads, C::kLoadsB>& L, char* slot, int64_t k0, int64_t K, bool on) {
-  static_assert(kCount <= C::kBI * C::kBJ, "more loads than MFMAs to spread them over");
+  // loads after each MFMA: one, or more where a tile has fewer MFMAs than loads
+  constexpr int kEach = (kCount + C::kBI * C::kBJ - 1) / (C::kBI * C::kBJ);
 #pragma unroll
   for (int q = 0; q < C::kBI * C::kBJ; ++q) {
     const int i = q / C::kBJ, j = q % C::kBJ;
     acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[j], fa[i], acc[i][j], 0, 0, 0);
-    if (q < kCount && on) issue_one<kB, kCheck>(L, slot, k0, K, kFirst + q);  // t is a constant once unrolled
+#pragma unroll
+    for (int e = q * kEach; e < (q + 1) * kEach; ++e)
+      if (e < kCount && on) issue_one<kB, kCheck>(L, slot, k0, K, kFirst + e);  // t is a constant once unrolled
   }
 }
 
@@ -1228,13 +1238,27 @@ MXQ_DEVICE void pp_tiles(const GemmArgs& p, char* lds) {
 
 // The four-wave kernels: one tile per workgroup.
 template <class C, int kEpi, int kOut>
-MXQ_DEVICE void four_wave_tile(const GemmArgs& p, char* lds) {
+MXQ_DEVICE void four_wave_tile(GemmArgs p, char* lds) {
   constexpr int kBM = C::kBM, kBN = C::kBN, kWaveM = C::kWaveM, kWaveN = C::kWaveN;
   constexpr int kBI = C::kBI, kBJ = C::kBJ, kSlotBytes = C::kSlotBytes, kLoads = C::kLoads;
   constexpr int kSlots = C::kSlots, kAhead = C::kAhead;
   constexpr int kStageLoads = C::kLoads + C::kLoadsB;  // loads per wave per stage (A and B chunks)
-  const int pos = pick_tile(p, p.tiles_m * p.tiles_n, lds);
-  if (pos < 0) return;
+  constexpr int kLoads0 = (kLoads + 1) / 2;            // A loads spread over K-step 0 (the rest over K-step 1)
+  int pos;
+  int64_t k_first = 0, k_len = p.K;  // this workgroup's K range
+  if constexpr (kEpi == kEpiSplit) {
+    // slice by slice, each in tile order: the workgroups of an XCD share a slice's operand panels
+    const int tiles = p.tiles_m * p.tiles_n;
+    const int t = static_position(blockIdx.x, tiles * p.splits);
+    const int slice = t / tiles;
+    pos = t - slice * tiles;
+    k_first = slice * p.slice_k;
+    k_len = min(p.slice_k, p.K - k_first);
+    p.d = reinterpret_cast<char*>(p.d) + slice * p.slice_stride;
+  } else {
+    pos = pick_tile(p, p.tiles_m * p.tiles_n, lds);
+    if (pos < 0) return;
+  }
   int tm, tn;
   tile_walk(pos, p.tiles_m, p.tiles_n, p.group_m, tm, tn);
   const int64_t m0 = (int64_t)tm * kBM, n0 = (int64_t)tn * kBN;
@@ -1262,13 +1286,19 @@ MXQ_DEVICE void four_wave_tile(const GemmArgs& p, char* lds) {
     // and B_kt, reads (kt+1, 0), and spreads the loads of B_kt+D over those MFMAs (into A_kt's
     // slot). A chunk is thus requested D-1 to D stages before it is used, and no wave issues a
     // burst of loads while its matrix pipe sits idle.
-    const int ktiles = (int)((p.K + kBK - 1) / kBK);
+    const int ktiles = (int)((k_len + kBK - 1) / kBK);
     Loader<kLoads, C::kLoadsB> ld;
     make_loader(ld, p, m0, n0);
+    if constexpr (kEpi == kEpiSplit) {
+#pragma unroll
+      for (int t = 0; t < kLoads; ++t) ld.a[t] += k_first;
+#pragma unroll
+      for (int t = 0; t < C::kLoadsB; ++t) ld.b[t] += k_first;
+    }
     const int pre = min(ktiles, kAhead);  // stages requested before the loop
     for (int s = 0; s < pre; ++s) {
-      issue_slot<false>(ld, lds + 2 * s * kSlotBytes, (int64_t)s * kBK, p.K);
-      issue_slot<true>(ld, lds + (2 * s + 1) * kSlotBytes, (int64_t)s * kBK, p.K);
+      issue_slot<false>(ld, lds + 2 * s * kSlotBytes, (int64_t)s * kBK, k_len);
+      issue_slot<true>(ld, lds + (2 * s + 1) * kSlotBytes, (int64_t)s * kBK, k_len);
     }
     // wait for stage 0: every load but those of stages 1 .. pre-1 has completed
     static_for<kAhead>([&](auto P) {
@@ -1299,12 +1329,12 @@ MXQ_DEVICE void four_wave_tile(const GemmArgs& p, char* lds) {
       load_frags<C>(lane, cur_a, cur_b, wrow, wcol, 1, f1a, f1b);
       wait_lgkm<kBI + kBJ>();
       __builtin_amdgcn_sched_barrier(0);
-      mma_step_dma<C, false, 0, kLoads / 2, !kSteady>(f0a, f0b, acc, ld, lds + pa * kSlotBytes, k2, p.K, more2);
+      mma_step_dma<C, false, 0, kLoads0, !kSteady>(f0a, f0b, acc, ld, lds + pa * kSlotBytes, k2, k_len, more2);
       __builtin_amdgcn_sched_barrier(0);
       load_frags<C>(lane, cur_a, cur_b, wrow, wcol, 2, f0a, f0b);
       wait_lgkm<kBI + kBJ>();
       __builtin_amdgcn_sched_barrier(0);
-      mma_step_dma<C, false, kLoads / 2, kLoads / 2, !kSteady>(f1a, f1b, acc, ld, lds + pa * kSlotBytes, k2, p.K, more2);
+      mma_step_dma<C, false, kLoads0, kLoads - kLoads0, !kSteady>(f1a, f1b, acc, ld, lds + pa * kSlotBytes, k2, k_len, more2);
       __builtin_amdgcn_sched_barrier(0);
       load_frags<C>(lane, cur_a, cur_b, wrow, wcol, 3, f1a, f1b);
       wait_lgkm<kBI + kBJ>();
@@ -1333,14 +1363,14 @@ MXQ_DEVICE void four_wave_tile(const GemmArgs& p, char* lds) {
         load_frags<C>(lane, lds_addr + (uint32_t)(na * kSlotBytes), lds_addr + (uint32_t)(nb * kSlotBytes), wrow, wcol, 0, f0a, f0b);
       }
       __builtin_amdgcn_sched_barrier(0);
-      mma_step_dma<C, true, 0, C::kLoadsB, !kSteady>(f1a, f1b, acc, ld, lds + sa * kSlotBytes, k2, p.K, more2 && more1);
+      mma_step_dma<C, true, 0, C::kLoadsB, !kSteady>(f1a, f1b, acc, ld, lds + sa * kSlotBytes, k2, k_len, more2 && more1);
       __builtin_amdgcn_sched_barrier(0);
       sa = na;
     };
     // steady < ktiles always (ktiles >= 1): written as do-while, the tail is seen to run at least
     // once, so no path leaves the steady loop with fragment reads in flight straight into the
     // epilogue (whose register copies would otherwise race those reads).
-    const int steady = (int)max<int64_t>(p.K / kBK - kAhead, 0);  // iterations whose stage kt+D is full
+    const int steady = (int)max<int64_t>(k_len / kBK - kAhead, 0);  // iterations whose stage kt+D is full
     int kt = 0;
     for (; kt < steady; ++kt) iteration(kt, std::true_type{});
     do {
@@ -1353,14 +1383,16 @@ MXQ_DEVICE void four_wave_tile(const GemmArgs& p, char* lds) {
     barrier_no_drain();
   }
 
+  // (a slice's epilogue is the raw int32 one, at its own place in the workspace)
+  constexpr int kStoreEpi = kEpi == kEpiSplit ? kEpiI32 : kEpi;
   EpiFactors<kBI, kOut> f;
-  load_epi_factors<C, kEpi, kOut>(p, m0, n0, wrow, f);
-  gemm_epilogue<C, kEpi, kOut, 0, C::kEpiLds>(p, lds, acc, m0, n0, wrow, wcol, f, [](int) {});
+  load_epi_factors<C, kStoreEpi, kOut>(p, m0, n0, wrow, f);
+  gemm_epilogue<C, kStoreEpi, kOut, 0, C::kEpiLds>(p, lds, acc, m0, n0, wrow, wcol, f, [](int) {});
 }
 
-template <int kEpi, int kOut, int kT, bool kDeep, bool kPP, int kTN = kT>
-__global__ __launch_bounds__((TileCfg<kT, kDeep, kPP, kTN>::kThreads), (TileCfg<kT, kDeep, kPP, kTN>::kPerCu)) void gemm_i8_kernel(GemmArgs p) {
-  typedef TileCfg<kT, kDeep, kPP, kTN> C;
+template <int kEpi, int kOut, int kT, bool kDeep, bool kPP, int kTN = kT, int kTM = kT>
+__global__ __launch_bounds__((TileCfg<kT, kDeep, kPP, kTN, kTM>::kThreads), (TileCfg<kT, kDeep, kPP, kTN, kTM>::kPerCu)) void gemm_i8_kernel(GemmArgs p) {
+  typedef TileCfg<kT, kDeep, kPP, kTN, kTM> C;
   static_assert(kT == 256 || (kEpi != kEpiGelu && kEpi != kEpiSwiGLU), "table epilogues need the 160 KB ring");
   __shared__ __attribute__((aligned(16))) char lds[C::kLds];
   if constexpr (kPP)
@@ -1446,6 +1478,154 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int table, int64_t workspace_byt
   return g;
 }
 
+// ---- split K ----
+// Problems of few tiles leave most CUs idle while each tile's workgroup walks the whole of K alone,
+// bound by what one CU draws from its L2 (about 65 KB/us): a 77 x 5376 x 7168 product is 56 tiles of 56
+// serial stages. With room for the partial sums (the workspace beyond the tile-queue counters), K is
+// cut into slices so that tiles x slices fill the CUs, each slice's int32 sums go to the workspace
+// (plain stores: the kernel boundary publishes them to the other XCDs) and a second kernel adds
+// them and applies the epilogue. int32 sums do not depend on the order, so the outputs are those of the unsplit
+// kernel, bit for bit. Rows to 32 and 64 run 32- and 64-row tiles (a quarter and half of a 128-row
+// tile's activation traffic). Weights from HBM, us before and after: 77 x 5376 x 7168 27.8 -> 17.7,
+// 1 x 5376 x 14336 42.3 -> 18.9, 77 x 5376 x 14336 50.9 -> 26.2, 333 x 5376 x 14336 52.3 -> 44.3,
+// 128 x 5120 x 20480 90.7 -> 33.1, 2 x 3072 x 3072 12.5 -> 8.1.
+struct SplitPlan {
+  int splits;       // slices; 0: no split
+  int tile_m;       // tile rows: 128, 64 or 32 (columns: 128)
+  int64_t slice_k;  // K-bytes per slice, a multiple of kBK
+  int64_t ldp;      // int32 per workspace row (a multiple of 4, so that rows stay 16-byte aligned)
+  int64_t bytes;    // workspace of the partial sums
+};
+
+// The slice count with the least estimated time, if that is below the unsplit kernel's. A workgroup
+// alone on its CU takes t_stage per stage (0.53 us on 128-row tiles, 0.41 and 0.28 on 64 and 32; 0.57 for the
+// unsplit kernel's), slowed by the weights' arrival from HBM (half of NK at 5.3 MB/us); the second
+// launch and the two fills add 5.5 us, each slice 0.5 us, and its sums are written and read once (7
+// MB/us). Measured over K = 3072 to 20480, M = 1 to 512 and 2 to 12 slices, the estimate picks a slice
+// count within a tenth of the best one's time and leaves alone what gains nothing (128 x 3072 x
+// 3072: 13.1 us unsplit, 13.2 at best split; 256 x 3072 x 3072 13.1 and 15.4).
+// SwiGLU (kTableSwiGLU): unsplit it runs 256-row tiles (1.5 us a stage), so even one slice of a
+// few rows, with the SwiGLU in the second kernel, is faster.
+static SplitPlan split_plan(int64_t M, int64_t N, int64_t K, int table) {
+  SplitPlan best{0, 0, 0, 0, 0};
+  const int64_t cus = std::min(mxq_cu_count(), 256);
+  const int tile_m = M <= 32 ? 32 : M <= 64 ? 64 : 128;
+  const int64_t tiles = ((M + tile_m - 1) / tile_m) * ((N + 127) / 128);
+  if (table == kTableGelu || tiles > cus) return best;
+  const int64_t stages = (K + kBK - 1) / kBK, ldp = (N + 3) / 4 * 4;
+  const double t_stage = tile_m == 32 ? 0.28 : tile_m == 64 ? 0.41 : 0.53;
+  double least = 0.95 * (double)stages * (table == kTableSwiGLU ? 1.5 : 0.57);
+  for (int64_t n = table == kTableSwiGLU ? 1 : 2; n <= std::min(cus / tiles, stages); ++n) {
+    const int64_t per = (stages + n - 1) / n;
+    if ((stages + per - 1) / per != n) continue;  // the same slices as a smaller count
+    const double t = (double)per * t_stage + (double)N * (double)K / 10.6e6 + 5.5 + 0.5 * (double)n + (double)(n * M * ldp) * 8 / 7e6;
+    if (t < least) {
+      least = t;
+      best = SplitPlan{(int)n, tile_m, per * kBK, ldp, n * M * ldp * 4};
+    }
+  }
+  return best;
+}
+
+// Sums the slices' partial results of four consecutive columns per thread and applies the epilogue.
+template <int kEpi, int kOut>
+__global__ __launch_bounds__(256) void split_reduce_kernel(GemmArgs p, const int32_t* __restrict__ part, int64_t ldp) {
+  constexpr int kElem = (kEpi == kEpiI32 || kOut == 0) ? 4 : 2;
+  const int64_t nout = kEpi == kEpiSwiGLU ? p.N / 2 : p.N;
+  const int groups = (int)((nout + 3) / 4);
+  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t row = idx / groups;
+  if (row >= p.M) return;
+  const int64_t col = (idx - row * groups) * 4;
+  auto sum = [&](int64_t c) {
+    v4i acc = {0, 0, 0, 0};
+    const int32_t* src = part + row * ldp + c;
+#pragma unroll 4
+    for (int s = 0; s < p.splits; ++s) acc += *reinterpret_cast<const v4i*>(src + s * (p.slice_stride / 4));
+    return v16i{acc[0], acc[1], acc[2], acc[3]};
+  };
+  auto run = [&](int64_t c, uint32_t* w) {
+    const v16i acc = sum(c);
+    float ws[4] = {}, bias[4] = {}, xs = 0.0f;
+    if constexpr (kEpi != kEpiI32) {
+      typedef typename OutT<kOut>::T BT;
+      xs = p.xs[row];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int64_t n = min(c + e, p.N - 1);
+        ws[e] = p.ws[p.ws_per_channel ? n : 0];
+        bias[e] = p.bias ? OutT<kOut>::load(reinterpret_cast<const BT*>(p.bias) + n) : -0.0f;
+      }
+    }
+    epi_run<kEpi, kOut>(acc, 0, xs, ws, bias, w);
+  };
+  uint32_t w[4];
+  if constexpr (kEpi == kEpiSwiGLU) {
+    // h columns col .. col + 3: gate columns of 32-column block col / 16, the matching up columns 16 further
+    const int64_t t = col / 16 * 32 + col % 16;
+    uint32_t g[2], u[2];
+    run(t, g);
+    run(t + 16, u);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      uint32_t h[2];
+#pragma unroll
+      for (int f = 0; f < 2; ++f) {
+        const float v = bf16_to_f32(silu_bf16((g[e] >> (16 * f)) & 0xFFFFu)) * bf16_to_f32((u[e] >> (16 * f)) & 0xFFFFu);
+        h[f] = v != v ? 0x7FC0u : f32_to_bf16_bits(v);
+      }
+      w[e] = h[0] | (h[1] << 16);
+    }
+  } else {
+    run(col, w);
+  }
+  if constexpr (kEpi == kEpiGatedRes) {
+    const int64_t gr = p.gate_rows[row];
+    const int64_t grow = gr < 0 ? (int64_t)0 : (gr >= p.gate_count ? p.gate_count - 1 : gr);
+    uint16_t* res = p.res + row * p.ldr + col;
+    const uint16_t* gate = p.gate + grow * p.ldg + col;
+    if (p.vec_store && col + 4 <= p.N) {
+      const v2u r = *reinterpret_cast<const v2u*>(res), g = *reinterpret_cast<const v2u*>(gate);
+      *reinterpret_cast<v2u*>(res) = v2u{gated_pair(r[0], w[0], g[0]), gated_pair(r[1], w[1], g[1])};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (col + e < p.N)
+          res[e] = (uint16_t)gated_pair(res[e], (w[e >> 1] >> (16 * (e & 1))) & 0xFFFFu, gate[e]);
+    }
+  } else {
+    store_run<kElem>(p.d, p.ldd, row, col, nout, p.vec_store && col + 4 <= nout, w);
+  }
+}
+
+template <int kEpi, int kOut>
+static int launch_split(GemmArgs args, const SplitPlan& s, void* workspace, hipStream_t stream) {
+  char* part = reinterpret_cast<char*>(workspace) + MXQ_GEMM_WORKSPACE_BYTES;
+  GemmArgs g = args;
+  g.d = part;
+  g.ldd = s.ldp;
+  g.vec_store = g.line_store = 1;
+  g.splits = args.splits = s.splits;
+  g.slice_k = s.slice_k;
+  g.slice_stride = args.slice_stride = args.M * s.ldp * 4;
+  g.tiles_m = (int)((args.M + s.tile_m - 1) / s.tile_m);
+  g.tiles_n = (int)((args.N + 127) / 128);
+  g.group_m = g.tiles_m;
+  const unsigned grid = (unsigned)(g.tiles_m * g.tiles_n * s.splits);
+  if (s.tile_m == 32)
+    gemm_i8_kernel<kEpiSplit, 0, 128, true, false, 128, 32><<<grid, kGemmThreads, 0, stream>>>(g);
+  else if (s.tile_m == 64)
+    gemm_i8_kernel<kEpiSplit, 0, 128, true, false, 128, 64><<<grid, kGemmThreads, 0, stream>>>(g);
+  else
+    gemm_i8_kernel<kEpiSplit, 0, 128, true, false><<<grid, kGemmThreads, 0, stream>>>(g);
+  int rc = mxq_check_launch("gemm_i8_kernel");
+  if (rc) return rc;
+  const int64_t groups = ((kEpi == kEpiSwiGLU ? args.N / 2 : args.N) + 3) / 4;
+  split_reduce_kernel<kEpi, kOut><<<(unsigned)((args.M * groups + 255) / 256), 256, 0, stream>>>(
+      args, reinterpret_cast<const int32_t*>(part), s.ldp);
+  return mxq_check_launch("split_reduce_kernel");
+}
+
 template <int kEpi, int kOut>
 static int launch_gemm(const GemmArgs& args0, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
   GemmArgs args = args0;
@@ -1466,6 +1646,11 @@ static int launch_gemm(const GemmArgs& args0, void* workspace, int64_t workspace
   if (kEpi == kEpiGatedRes) {
     args.vec_store = args.vec_store && ((uintptr_t)args.gate % 8 == 0) && (args.ldg % 4 == 0);
     args.line_store = args.line_store && ((uintptr_t)args.gate % 16 == 0) && (args.ldg % 8 == 0);
+  }
+  if constexpr (kEpi != kEpiGelu) {
+    const SplitPlan sp = split_plan(args.M, args.N, args.K, kEpi == kEpiSwiGLU ? kTableSwiGLU : 0);
+    if (sp.splits && workspace && workspace_bytes >= MXQ_GEMM_WORKSPACE_BYTES + sp.bytes)
+      return launch_split<kEpi, kOut>(args, sp, workspace, stream);
   }
   const unsigned grid = (unsigned)g.grid;
   if constexpr (kEpi == kEpiSwiGLU) {
@@ -1512,6 +1697,14 @@ static int check_gemm_shape(const int8_t* a, const int8_t* b, const void* d, int
 }  // namespace mxq
 
 using namespace mxq;
+
+extern "C" int mxq_int8_gemm_workspace(int64_t M, int64_t N, int64_t K, int table_epilogue, int64_t* bytes) {
+  if (M < 0 || N < 0 || K < 0 || !bytes) return mxq_set_error(MXQ_ERR_INVALID, "bad GEMM workspace request");
+  if (table_epilogue < 0 || table_epilogue > kTableSwiGLU) return mxq_set_error(MXQ_ERR_INVALID, "table_epilogue must be 0, 1 or 2");
+  *bytes = MXQ_GEMM_WORKSPACE_BYTES;
+  if (M > 0 && N > 0 && K > 0) *bytes += split_plan(M, N, K, table_epilogue).bytes;
+  return MXQ_OK;
+}
 
 extern "C" int mxq_int8_gemm_plan(int64_t M, int64_t N, int64_t K, int table_epilogue,
                                   int64_t workspace_bytes, int64_t* plan) {

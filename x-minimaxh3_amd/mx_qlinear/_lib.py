@@ -8,6 +8,7 @@ is raised.
 from __future__ import annotations
 
 import ctypes
+import functools
 import pathlib
 import threading
 
@@ -38,6 +39,7 @@ SIGNATURES: dict[str, list] = {
     "mxq_adaln": [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _F, _P],
     "mxq_adaln_quantize_int8": [_P, _P, _P, _I64, _I64, _F, _P, _P, _P, _I64, _I64, _P],
     "mxq_int8_gemm_plan": [_I64, _I64, _I64, _I, _I64, _P],
+    "mxq_int8_gemm_workspace": [_I64, _I64, _I64, _I, _P],
     "mxq_int8_gemm_i32": [_P, _P, _P, _I64, _I64, _I64, _I64, _P, _I64, _P],
     "mxq_int8_gemm_dequant": [_P, _P, _P, _P, _I64, _P, _P, _I64, _I64, _I64, _I64, _I, _P, _I64, _P],
     "mxq_int8_gemm_dequant_gelu_absmax": [_P, _P, _P, _P, _I64, _P, _P, _P, _I64, _I64, _I64, _I64, _P, _I64,
@@ -110,6 +112,15 @@ def gemm_plan(m: int, n: int, k: int, table: int = 0, workspace_bytes: int = GEM
     call("mxq_int8_gemm_plan", m, n, k, int(table), workspace_bytes, out)
     return {"tile": out[0], "grid": out[1], "tiles": out[2], "pool": out[3], "wg_per_xcd": out[4],
             "ahead": out[5], "group_m": out[6], "persistent": bool(out[7]), "tile_n": out[8]}
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_workspace_bytes(m: int, n: int, k: int, table: int = 0) -> int:
+    """Workspace an INT8 GEMM of this shape can use (mxq_int8_gemm_workspace): the tile-queue counters
+    alone, or with room for the partial sums of a K split."""
+    out = ctypes.c_int64()
+    call("mxq_int8_gemm_workspace", m, n, k, int(table), ctypes.byref(out))
+    return out.value
 
 
 def call(name: str, *args) -> None:

@@ -32,15 +32,25 @@ def _stream(device: torch.device):
 _GEMM_WORKSPACES: dict[tuple[int, int], torch.Tensor] = {}
 
 
-def _gemm_ws(device: torch.device):
-    """The INT8 GEMMs' tile-queue workspace for the current stream on ``device``, as the two
+def _gemm_ws(device: torch.device, m: int = 0, n: int = 0, k: int = 0, table: int = 0):
+    """The workspace of an INT8 GEMM of this shape on ``device``'s current stream, as the two
     trailing arguments (pointer, bytes) the GEMM entry points take before the stream: the
     counters with which the XCDs share out the last tiles at run time. One zero-filled workspace
     per (device, stream), made on that stream's first GEMM and kept for the process, as the
     reference keeps one per (device, stream) inside its launchers
     (CK/backends/cuda/ops/cutlass_gemm_int8.cu:39-55); the kernels leave it zero after every call.
-    Under graph capture no workspace is passed (the static tile order, the same outputs), so a
-    captured graph shares no memory with eager calls."""
+    Under graph capture no such workspace is passed (the static tile order, the same outputs), so a
+    captured graph shares no memory with eager calls.
+
+    A problem of few tiles, whose K the library splits, gets room for its partial sums instead: a
+    tensor of this call's own (it uses no counters), which the returned pointer keeps alive until the
+    launch."""
+    need = _lib.gemm_workspace_bytes(m, n, k, table)
+    if need > _lib.GEMM_WORKSPACE_BYTES:
+        part = torch.empty(need, dtype=torch.uint8, device=device)
+        ptr = _p(part)
+        ptr.keep = part
+        return ptr, need
     with torch.cuda.device(device):
         if torch.cuda.is_current_stream_capturing():
             return None, 0
@@ -466,7 +476,7 @@ def mm_int8(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
     a2, w2 = _gemm_activation(a.contiguous(), kp), _gemm_weight(b, kp, transpose=True)
     k = kp
     with torch.cuda.device(dev):
-        call("mxq_int8_gemm_i32", _p(a2), _p(w2), _p(out), m, n, k, n, *_gemm_ws(dev), _stream(dev))
+        call("mxq_int8_gemm_i32", _p(a2), _p(w2), _p(out), m, n, k, n, *_gemm_ws(dev, m, n, k), _stream(dev))
     return out
 
 
@@ -548,7 +558,7 @@ def int8_linear_prequantized(x_qdata: torch.Tensor, x_scale: torch.Tensor, weigh
     q2, w2, k = _pad_k(x_qdata.contiguous(), weight)
     with torch.cuda.device(dev):
         call("mxq_int8_gemm_dequant", _p(q2), _p(w2), _p(xs), _p(ws), ws.numel(), _p(b), _p(out),
-             m, n, k, n, code, *_gemm_ws(dev), _stream(dev))
+             m, n, k, n, code, *_gemm_ws(dev, m, n, k), _stream(dev))
     return out
 
 
@@ -664,23 +674,22 @@ def int8_ffn_gelu(x: torch.Tensor, fc1_weight: torch.Tensor, fc1_scale: torch.Te
     w1 = _gemm_weight(fc1_weight, k)
     w2 = _gemm_weight(fc2_weight, hidden)
     st = _stream(dev)
-    gws = _gemm_ws(dev)
     with torch.cuda.device(dev):
         call("mxq_quantize_int8_rowwise", _p(x2), _OUT_CODES[x.dtype], _p(ws.xq), _p(ws.xs), m, k,
              _lib.ACT_NONE, st)
         if hidden <= _GELU_QUANT_MAX_COLS:
             call("mxq_int8_gemm_dequant", _p(ws.xq), _p(w1), _p(ws.xs), _p(s1), s1.numel(), _p(b1),
-                 _p(ws.h), m, hidden, k, hidden, _lib.DTYPE_BF16, *gws, st)
+                 _p(ws.h), m, hidden, k, hidden, _lib.DTYPE_BF16, *_gemm_ws(dev, m, hidden, k), st)
             call("mxq_quantize_int8_rowwise_gelu", _p(ws.h), _p(ws.h) if return_hidden else None,
                  _p(ws.hq), _p(ws.hs), m, hidden, st)
         else:
             call("mxq_fill_f32", _p(ws.hmax), 0.0, m, st)
             call("mxq_int8_gemm_dequant_gelu_absmax", _p(ws.xq), _p(w1), _p(ws.xs), _p(s1), s1.numel(),
-                 _p(b1), _p(ws.h), _p(ws.hmax), m, hidden, k, hidden, *gws, st)
+                 _p(b1), _p(ws.h), _p(ws.hmax), m, hidden, k, hidden, *_gemm_ws(dev), st)
             call("mxq_quantize_int8_rowwise_absmax", _p(ws.h), _p(ws.hmax), _p(ws.hq), _p(ws.hs), m,
                  hidden, st)
         call("mxq_int8_gemm_dequant", _p(ws.hq), _p(w2), _p(ws.hs), _p(s2), s2.numel(), _p(b2),
-             _p(out), m, n, hidden, n, _lib.DTYPE_BF16, *gws, st)
+             _p(out), m, n, hidden, n, _lib.DTYPE_BF16, *_gemm_ws(dev, m, n, hidden), st)
     out = out.reshape(*x.shape[:-1], n)
     return (out, ws.h.reshape(*x.shape[:-1], hidden)) if return_hidden else out
 
@@ -797,7 +806,7 @@ def int8_linear_gated_residual_(residual: torch.Tensor, x: torch.Tensor, weight:
     q2, w2, k = _pad_k(q, weight)
     with torch.cuda.device(dev):
         call("mxq_int8_gemm_gated_residual", _p(q2), _p(w2), _p(xs), _p(ws), ws.numel(), _p(b), _p(res2),
-             res2.stride(0), _p(g), g.stride(0), g.shape[0], _p(gr), rows, n, k, *_gemm_ws(dev), _stream(dev))
+             res2.stride(0), _p(g), g.stride(0), g.shape[0], _p(gr), rows, n, k, *_gemm_ws(dev, rows, n, k), _stream(dev))
     return residual
 
 
@@ -877,7 +886,7 @@ def int8_swiglu_fc1(x_qdata: torch.Tensor, x_scale: torch.Tensor, fc1: PreparedS
     q2, w2, k = _pad_k(x_qdata.contiguous(), fc1.qweight)
     with torch.cuda.device(dev):
         call("mxq_int8_gemm_dequant_swiglu", _p(q2), _p(w2), _p(xs), _p(fc1.scale), fc1.scale.numel(),
-             _p(fc1.bias), _p(h), m, n2, k, h.stride(0), *_gemm_ws(dev), _stream(dev))
+             _p(fc1.bias), _p(h), m, n2, k, h.stride(0), *_gemm_ws(dev, m, n2, k, 2), _stream(dev))
     return h
 
 
@@ -1008,7 +1017,7 @@ def w4a8_int8_linear(x: torch.Tensor, qdata: torch.Tensor, s_rel: torch.Tensor, 
     work = torch.empty((chunk, k), dtype=torch.int8, device=dev)
     with torch.cuda.device(dev):
         call("mxq_w4a8_codebook_gemm", _p(xq), _p(qdata.contiguous()), _p(sr), scode, _p(cb), _p(sch),
-             _p(xs), _p(b), _p(work), _p(out), m, n, k, group_size, chunk, code, *_gemm_ws(dev), _stream(dev))
+             _p(xs), _p(b), _p(work), _p(out), m, n, k, group_size, chunk, code, *_gemm_ws(dev, m, min(chunk, n), k), _stream(dev))
         if correction is not None:
             sx = torch.empty((m, k // group_size), dtype=out_dtype, device=dev)
             call("mxq_int8_group_sums", _p(xq), _p(xs), _p(sx), m, k, group_size, code, _stream(dev))
