@@ -139,11 +139,12 @@ int mxq_adaln_quantize_int8_f16(const void* x, const void* scale, const void* sh
 #define MXQ_GEMM_WORKSPACE_BYTES ((int64_t)4096)
 
 /*
- * The workspace an M x N x K GEMM can use, in *bytes: MXQ_GEMM_WORKSPACE_BYTES, plus room for the
- * partial sums of a problem of so few tiles that the library would cut its K into slices to fill the CUs
- * (table_epilogue as in mxq_int8_gemm_plan). Such a problem given that much runs two launches,
- * the slices and their sum with the epilogue; given less it runs unsplit, with the same outputs. The bytes
- * behind the first MXQ_GEMM_WORKSPACE_BYTES need no initial value and are left with any.
+ * The workspace an M x N x K GEMM can use, in *bytes (table_epilogue as in mxq_int8_gemm_plan): 0 if
+ * none, MXQ_GEMM_WORKSPACE_BYTES for the tile queue, or that plus room for the partial sums of a problem
+ * of so few tiles that the library would cut its K into slices to fill the CUs. Such a problem given that
+ * much runs two launches, the slices and their sum with the epilogue; given less it runs unsplit, with the
+ * same outputs. It uses no counters, and the bytes behind the first MXQ_GEMM_WORKSPACE_BYTES need no
+ * initial value and are left with any.
  */
 int mxq_int8_gemm_workspace(int64_t M, int64_t N, int64_t K, int table_epilogue, int64_t* bytes);
 

@@ -1701,8 +1701,13 @@ using namespace mxq;
 extern "C" int mxq_int8_gemm_workspace(int64_t M, int64_t N, int64_t K, int table_epilogue, int64_t* bytes) {
   if (M < 0 || N < 0 || K < 0 || !bytes) return mxq_set_error(MXQ_ERR_INVALID, "bad GEMM workspace request");
   if (table_epilogue < 0 || table_epilogue > kTableSwiGLU) return mxq_set_error(MXQ_ERR_INVALID, "table_epilogue must be 0, 1 or 2");
-  *bytes = MXQ_GEMM_WORKSPACE_BYTES;
-  if (M > 0 && N > 0 && K > 0) *bytes += split_plan(M, N, K, table_epilogue).bytes;
+  *bytes = 0;
+  if (M == 0 || N == 0 || K == 0) return MXQ_OK;
+  const SplitPlan s = split_plan(M, N, K, table_epilogue);
+  if (s.splits)
+    *bytes = MXQ_GEMM_WORKSPACE_BYTES + s.bytes;
+  else if (plan_gemm(M, N, table_epilogue, MXQ_GEMM_WORKSPACE_BYTES).pool)
+    *bytes = MXQ_GEMM_WORKSPACE_BYTES;
   return MXQ_OK;
 }
 

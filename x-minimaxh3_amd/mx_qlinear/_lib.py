@@ -116,8 +116,8 @@ def gemm_plan(m: int, n: int, k: int, table: int = 0, workspace_bytes: int = GEM
 
 @functools.lru_cache(maxsize=4096)
 def gemm_workspace_bytes(m: int, n: int, k: int, table: int = 0) -> int:
-    """Workspace an INT8 GEMM of this shape can use (mxq_int8_gemm_workspace): the tile-queue counters
-    alone, or with room for the partial sums of a K split."""
+    """Workspace an INT8 GEMM of this shape can use (mxq_int8_gemm_workspace): none, the tile-queue
+    counters, or those with room for the partial sums of a K split."""
     out = ctypes.c_int64()
     call("mxq_int8_gemm_workspace", m, n, k, int(table), ctypes.byref(out))
     return out.value
@@ -125,7 +125,7 @@ def gemm_workspace_bytes(m: int, n: int, k: int, table: int = 0) -> int:
 
 def call(name: str, *args) -> None:
     """Call ``name``; translate a non-zero return code into an exception."""
-    lib = load()
+    lib = _lib or load()
     rc = getattr(lib, name)(*args)
     if rc != MXQ_OK:
         msg = lib.mxq_last_error().decode(errors="replace")

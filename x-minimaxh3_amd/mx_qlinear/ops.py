@@ -29,6 +29,40 @@ def _stream(device: torch.device):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
+# The host side of a call is part of a small call's time (a few rows through one layer: two or three
+# kernels of 4 to 20 us), so the launches below take what the tensors already are: pointers go to ctypes as
+# plain integers, the raw stream handle is read without building a Stream object, the device is switched
+# only when it is not the current one, and a factor that is already float32 (or the output dtype),
+# contiguous and in place passes through without a chain of no-op conversions. One int8_linear of two
+# launches: 41 -> 20 us of host time (one row 24 -> 16, the row quantizer alone 15 -> 9).
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
+
+def _ptr(t: torch.Tensor | None):
+    return None if t is None else t.data_ptr()
+
+
+def _launch(device: torch.device, name: str, *args) -> None:
+    """``name`` with ``device`` current, its current stream appended to the arguments."""
+    if torch.cuda.current_device() == device.index:
+        call(name, *args, _raw_stream(device.index))
+    else:
+        with torch.cuda.device(device):
+            call(name, *args, _raw_stream(device.index))
+
+
+def _rows(x: torch.Tensor, width: int) -> torch.Tensor:
+    """``x`` as contiguous ``[rows, width]``."""
+    return x if x.dim() == 2 and x.is_contiguous() else x.reshape(-1, width).contiguous()
+
+
+def _vector(t: torch.Tensor, dtype: torch.dtype, dev: torch.device) -> torch.Tensor:
+    """``t`` in ``dtype`` on ``dev``, contiguous; its shape is left as it is (kernels take a pointer)."""
+    if t.dtype == dtype and t.device == dev and t.is_contiguous():
+        return t
+    return t.to(device=dev, dtype=dtype).contiguous()
+
+
 _GEMM_WORKSPACES: dict[tuple[int, int], torch.Tensor] = {}
 
 
@@ -45,22 +79,24 @@ def _gemm_ws(device: torch.device, m: int = 0, n: int = 0, k: int = 0, table: in
     A problem of few tiles, whose K the library splits, gets room for its partial sums instead: a
     tensor of this call's own (it uses no counters), which the returned pointer keeps alive until the
     launch."""
-    need = _lib.gemm_workspace_bytes(m, n, k, table)
-    if need > _lib.GEMM_WORKSPACE_BYTES:
-        part = torch.empty(need, dtype=torch.uint8, device=device)
-        ptr = _p(part)
-        ptr.keep = part
-        return ptr, need
+    if m:
+        need = _lib.gemm_workspace_bytes(m, n, k, table)
+        if need == 0:  # neither a queue nor a split
+            return None, 0
+        if need > _lib.GEMM_WORKSPACE_BYTES:
+            part = torch.empty(need, dtype=torch.uint8, device=device)
+            ptr = _p(part)
+            ptr.keep = part
+            return ptr, need
     with torch.cuda.device(device):
         if torch.cuda.is_current_stream_capturing():
             return None, 0
-    stream = torch.cuda.current_stream(device)
-    key = (device.index, stream.cuda_stream)
+    key = (device.index, _raw_stream(device.index))
     ws = _GEMM_WORKSPACES.get(key)
     if ws is None:
         ws = torch.zeros(_lib.GEMM_WORKSPACE_BYTES, dtype=torch.uint8, device=device)
         _GEMM_WORKSPACES[key] = ws
-    return _p(ws), ws.numel()
+    return _p(ws), _lib.GEMM_WORKSPACE_BYTES
 
 
 def _require_gpu(*tensors: torch.Tensor | None) -> torch.device:
@@ -133,13 +169,12 @@ def quantize_int8_rowwise(x: torch.Tensor, stochastic_rounding: int | None = 0,
     k = x.shape[-1]
     if k == 0:
         raise ValueError("quantize_int8_rowwise needs a non-empty last dimension")
-    x2 = x.reshape(-1, k).contiguous()
+    x2 = _rows(x, k)
     m = x2.shape[0]
     q = torch.empty((m, k), dtype=torch.int8, device=dev)
     s = torch.empty((m, 1), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        call("mxq_quantize_int8_rowwise", _p(x2), _OUT_CODES[x.dtype], _p(q), _p(s), m, k, act, _stream(dev))
-    return q.reshape(x.shape), s.reshape(*x.shape[:-1], 1)
+    _launch(dev, "mxq_quantize_int8_rowwise", _ptr(x2), _OUT_CODES[x.dtype], _ptr(q), _ptr(s), m, k, act)
+    return (q, s) if x.dim() == 2 else (q.reshape(x.shape), s.reshape(*x.shape[:-1], 1))
 
 
 def _quantize_int8_rowwise_stochastic(x: torch.Tensor, seed: int) -> tuple[torch.Tensor, torch.Tensor]:
@@ -191,15 +226,14 @@ def quantize_int8_rowwise_convrot(x: torch.Tensor, group_size: int = 256,
         raise ValueError(f"ConvRot group size {group_size} does not divide input features {k}")
     if k % 16:
         raise NotImplementedError(f"the rotation quantizer needs a multiple of 16 columns, got {k}")
-    x2 = x.reshape(-1, width).contiguous()
+    x2 = _rows(x, width)
     m = x2.shape[0]
     q = torch.empty((m, k), dtype=torch.int8, device=dev)
     s = torch.empty((m, 1), dtype=torch.float32, device=dev)
     if m:
-        with torch.cuda.device(dev):
-            call("mxq_quantize_int8_rowwise_convrot", _p(x2), _OUT_CODES[x.dtype], _p(q), _p(s), m, k,
-                 group_size, act, _stream(dev))
-    return q.reshape(*x.shape[:-1], k), s.reshape(*x.shape[:-1], 1)
+        _launch(dev, "mxq_quantize_int8_rowwise_convrot", _ptr(x2), _OUT_CODES[x.dtype], _ptr(q), _ptr(s), m, k,
+                group_size, act)
+    return (q, s) if x.dim() == 2 else (q.reshape(*x.shape[:-1], k), s.reshape(*x.shape[:-1], 1))
 
 
 def quantize_int8_convrot_weight(weight: torch.Tensor, group_size: int = 256) -> tuple[torch.Tensor, torch.Tensor]:
@@ -252,10 +286,10 @@ def apply_input_act(x: torch.Tensor, input_act: str | None) -> torch.Tensor:
 
 
 def _modulation(t: torch.Tensor, rows: int, cols: int, dev, name: str, dtype=torch.bfloat16):
-    t = t.to(device=dev, dtype=dtype)
+    t = _vector(t, dtype, dev)
     if t.shape[-1] != cols:
         raise ValueError(f"{name} last dimension {t.shape[-1]} != {cols}")
-    t2 = t.reshape(-1, cols).contiguous()
+    t2 = _rows(t, cols)
     g = t2.shape[0]
     if g == 0 or rows % g != 0:
         raise ValueError(f"{name} with {g} rows does not broadcast over {rows} rows")
@@ -309,8 +343,7 @@ def adaln_quantize_int8(x: torch.Tensor, scale: torch.Tensor, shift: torch.Tenso
         sc, sg = _modulation(scale, rows, d, dev, "scale", x.dtype)
         sh, hg = _modulation(shift, rows, d, dev, "shift", x.dtype)
         entry = "mxq_adaln_quantize_int8_f16" if x.dtype == torch.float16 else "mxq_adaln_quantize_int8"
-        with torch.cuda.device(dev):
-            call(entry, _p(x2), _p(sc), _p(sh), sg, hg, float(eps), _p(q), _p(s), _p(y), rows, d, _stream(dev))
+        _launch(dev, entry, _ptr(x2), _ptr(sc), _ptr(sh), sg, hg, float(eps), _ptr(q), _ptr(s), _ptr(y), rows, d)
     out = (q.reshape(x.shape), s.reshape(*x.shape[:-1], 1))
     return out + (y.reshape(x.shape),) if return_modulated else out
 
@@ -319,7 +352,7 @@ def _norm_parts(norm, d: int, dev, dtype=torch.bfloat16) -> tuple[torch.Tensor, 
     """An RMSNorm module (``.weight`` [d], ``.eps``) or a ``(weight, eps)`` pair ->
     (weight on ``dev`` in x's dtype, eps); the weight is cast like ``weight.to(x.dtype)``."""
     weight, eps = (norm.weight, norm.eps) if hasattr(norm, "weight") else norm
-    w = weight.detach().to(device=dev, dtype=dtype).reshape(-1).contiguous()
+    w = _vector(weight.detach(), dtype, dev)
     if w.numel() != d:
         raise ValueError(f"RMSNorm weight has {w.numel()} entries, expected {d}")
     return w, float(eps)
@@ -331,7 +364,7 @@ def _segment_table(t: torch.Tensor, d: int, dev, name: str, dtype=torch.bfloat16
         t = t.reshape(1, -1)
     if t.dim() != 2 or t.shape[1] != d:
         raise ValueError(f"{name} must be [rows, {d}], got {tuple(t.shape)}")
-    return t.to(device=dev, dtype=dtype).contiguous()
+    return _vector(t, dtype, dev)
 
 
 def rms_adaln_quantize_int8(value: torch.Tensor, norm, shift: torch.Tensor, scale: torch.Tensor,
@@ -380,16 +413,14 @@ def _rms_adaln_call(value, norm, shift, scale, segments, quant: bool, group: int
     q = torch.empty((rows, d), dtype=torch.int8, device=dev) if quant else None
     s = torch.empty((rows, 1), dtype=torch.float32, device=dev) if quant else None
     if rows and d:
-        with torch.cuda.device(dev):
-            if x.dtype == torch.float16:
-                call("mxq_rms_adaln_quantize_int8_f16", _p(x), _p(w), _p(sc), _p(sh), sc.stride(0), sc.shape[0],
-                     _p(mr), eps, _p(y), _p(q), _p(s), rows, d, group if quant else 0, _stream(dev))
-            else:
-                # room for bf16(1 + scale) of each modulation row, formed once per call
-                ws = torch.empty(sc.shape[0] * sc.stride(0) * 2 if quant else 0, dtype=torch.uint8, device=dev)
-                call("mxq_rms_adaln_quantize_int8", _p(x), _p(w), _p(sc), _p(sh), sc.stride(0), sc.shape[0],
-                     _p(mr), eps, _p(y), _p(q), _p(s), rows, d, group if quant else 0, _p(ws), ws.numel(),
-                     _stream(dev))
+        args = (_ptr(x), _ptr(w), _ptr(sc), _ptr(sh), sc.stride(0), sc.shape[0], _ptr(mr), eps, _ptr(y), _ptr(q), _ptr(s),
+                rows, d, group if quant else 0)
+        if x.dtype == torch.float16:
+            _launch(dev, "mxq_rms_adaln_quantize_int8_f16", *args)
+        else:
+            # room for bf16(1 + scale) of each modulation row, formed once per call
+            ws = torch.empty(sc.shape[0] * sc.stride(0) * 2 if quant else 0, dtype=torch.uint8, device=dev)
+            _launch(dev, "mxq_rms_adaln_quantize_int8", *args, _ptr(ws), ws.numel())
     if not quant:
         return y
     return (q, s, y) if want_y else (q, s)
@@ -481,7 +512,7 @@ def mm_int8(a: torch.Tensor, b: torch.Tensor) -> torch.Tensor:
 
 
 def _weight_scale(weight_scale: torch.Tensor, n: int, dev) -> torch.Tensor:
-    ws = torch.as_tensor(weight_scale).to(device=dev, dtype=torch.float32).reshape(-1).contiguous()
+    ws = _vector(torch.as_tensor(weight_scale), torch.float32, dev)
     if ws.numel() not in (1, n):
         raise ValueError(
             f"INT8 weight scale must be scalar or per-output-channel, got {tuple(weight_scale.shape)} "
@@ -493,7 +524,7 @@ def _weight_scale(weight_scale: torch.Tensor, n: int, dev) -> torch.Tensor:
 def _bias(bias: torch.Tensor | None, n: int, dtype: torch.dtype, dev):
     if bias is None:
         return None
-    b = bias.to(device=dev, dtype=dtype).reshape(-1).contiguous()
+    b = _vector(bias, dtype, dev)
     if b.numel() != n:
         raise ValueError(f"bias has {b.numel()} entries, expected {n}")
     return b
@@ -543,22 +574,26 @@ def int8_linear_prequantized(x_qdata: torch.Tensor, x_scale: torch.Tensor, weigh
     code = _out_code(out_dtype)
     ws = _weight_scale(weight_scale, n, dev)
     b = _bias(bias, n, out_dtype, dev)
-    xs = x_scale.to(device=dev, dtype=torch.float32).reshape(-1).contiguous()
+    xs = _vector(x_scale, torch.float32, dev)
     if xs.numel() != m:
         raise ValueError(f"x_scale has {xs.numel()} entries, expected {m}")
+    return _gemm_dequant(x_qdata, xs, weight, ws, b, out_dtype, code, dev)
+
+
+def _gemm_dequant(x_qdata, xs, weight, ws, b, out_dtype, code, dev) -> torch.Tensor:
+    """The GEMM (or one-row GEMV) of :func:`int8_linear_prequantized` from checked factors."""
+    m, n, k = x_qdata.shape[0], weight.shape[0], x_qdata.shape[1]
     out = torch.empty((m, n), dtype=out_dtype, device=dev)
     if m == 0 or n == 0:
         return out
-    k = x_qdata.shape[1]
     if m == 1 and _m1_ok(k):
-        with torch.cuda.device(dev):
-            call("mxq_int8_gemv_dequant", _p(_aligned16(x_qdata)), _p(xs), _p(_gemm_weight(weight, k)), _p(ws),
-                 ws.numel(), _p(b), _p(out), n, k, code, _stream(dev))
+        xq, w2 = _aligned16(x_qdata), _gemm_weight(weight, k)
+        _launch(dev, "mxq_int8_gemv_dequant", _ptr(xq), _ptr(xs), _ptr(w2), _ptr(ws), ws.numel(), _ptr(b), _ptr(out), n, k,
+                code)
         return out
     q2, w2, k = _pad_k(x_qdata.contiguous(), weight)
-    with torch.cuda.device(dev):
-        call("mxq_int8_gemm_dequant", _p(q2), _p(w2), _p(xs), _p(ws), ws.numel(), _p(b), _p(out),
-             m, n, k, n, code, *_gemm_ws(dev, m, n, k), _stream(dev))
+    _launch(dev, "mxq_int8_gemm_dequant", _ptr(q2), _ptr(w2), _ptr(xs), _ptr(ws), ws.numel(), _ptr(b), _ptr(out),
+            m, n, k, n, code, *_gemm_ws(dev, m, n, k))
     return out
 
 
@@ -587,31 +622,32 @@ def int8_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tenso
             raise ValueError(f"ConvRot group size {convrot_groupsize} does not divide input features {width}")
     dev = _require_gpu(x, weight)
     n = weight.shape[0]
-    _weight_scale(weight_scale, n, dev)  # validate before launching anything
+    ws = _weight_scale(weight_scale, n, dev)  # validate before launching anything
     if act and x.dtype == torch.float32:
         raise NotImplementedError(f"input_act={input_act!r} needs a bfloat16 or float16 input")
     lead = x.shape[:-1]
     if x.numel() == 0:
         return torch.empty((*lead, n), dtype=out_dtype, device=dev)
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     if x2.shape[0] == 1 and x.dtype == torch.bfloat16 and _m1_ok(width) and n:
         # one token: the row quantizer, then the weight-streaming GEMV (int8_linear_m1's route)
-        ws = _weight_scale(weight_scale, n, dev)
         b = _bias(bias, n, out_dtype, dev)
         out = torch.empty((1, n), dtype=out_dtype, device=dev)
         xq = torch.empty((1, width), dtype=torch.int8, device=dev)
         xs = torch.empty((1, 1), dtype=torch.float32, device=dev)
-        with torch.cuda.device(dev):
-            call("mxq_int8_linear_m1", _p(_aligned16(x2)), _p(_gemm_weight(weight, width)), _p(ws), ws.numel(), _p(b),
-                 _p(out), n, width, convrot_groupsize if convrot else 0, act, _out_code(out_dtype), _p(xq), _p(xs),
-                 _stream(dev))
-        return out.reshape(*lead, n)
+        x2, w2 = _aligned16(x2), _gemm_weight(weight, width)
+        _launch(dev, "mxq_int8_linear_m1", _ptr(x2), _ptr(w2), _ptr(ws), ws.numel(), _ptr(b),
+                _ptr(out), n, width, convrot_groupsize if convrot else 0, act, _out_code(out_dtype), _ptr(xq), _ptr(xs))
+        return out if x.dim() == 2 else out.reshape(*lead, n)
     if convrot:
         q, s = quantize_int8_rowwise_convrot(x2, convrot_groupsize, input_act)
     else:
         q, s = quantize_int8_rowwise(x2, input_act=input_act)
-    out = int8_linear_prequantized(q, s, weight, weight_scale, bias, out_dtype)
-    return out.reshape(*lead, n)
+    if weight.dim() != 2 or weight.dtype != torch.int8:
+        raise ValueError("weight must be a 2-D int8 tensor")
+    code = _out_code(out_dtype)
+    out = _gemm_dequant(q, s, weight, ws, _bias(bias, n, out_dtype, dev), out_dtype, code, dev)
+    return out if x.dim() == 2 else out.reshape(*lead, n)
 
 
 # ---------------------------------------------------------------------------------------
@@ -660,7 +696,7 @@ def int8_ffn_gelu(x: torch.Tensor, fc1_weight: torch.Tensor, fc1_scale: torch.Te
         raise ValueError("FFN weight shapes do not chain")
     if k % 16 or hidden % 16:
         raise NotImplementedError("int8_ffn_gelu needs K and the hidden width to be multiples of 16")
-    x2 = x.reshape(-1, k).contiguous()
+    x2 = _rows(x, k)
     m = x2.shape[0]
     s1 = _weight_scale(fc1_scale, hidden, dev)
     s2 = _weight_scale(fc2_scale, n, dev)
@@ -673,23 +709,21 @@ def int8_ffn_gelu(x: torch.Tensor, fc1_weight: torch.Tensor, fc1_scale: torch.Te
     ws = workspace if reuse else FfnWorkspace(m, k, hidden, dev)
     w1 = _gemm_weight(fc1_weight, k)
     w2 = _gemm_weight(fc2_weight, hidden)
-    st = _stream(dev)
-    with torch.cuda.device(dev):
-        call("mxq_quantize_int8_rowwise", _p(x2), _OUT_CODES[x.dtype], _p(ws.xq), _p(ws.xs), m, k,
-             _lib.ACT_NONE, st)
-        if hidden <= _GELU_QUANT_MAX_COLS:
-            call("mxq_int8_gemm_dequant", _p(ws.xq), _p(w1), _p(ws.xs), _p(s1), s1.numel(), _p(b1),
-                 _p(ws.h), m, hidden, k, hidden, _lib.DTYPE_BF16, *_gemm_ws(dev, m, hidden, k), st)
-            call("mxq_quantize_int8_rowwise_gelu", _p(ws.h), _p(ws.h) if return_hidden else None,
-                 _p(ws.hq), _p(ws.hs), m, hidden, st)
-        else:
-            call("mxq_fill_f32", _p(ws.hmax), 0.0, m, st)
-            call("mxq_int8_gemm_dequant_gelu_absmax", _p(ws.xq), _p(w1), _p(ws.xs), _p(s1), s1.numel(),
-                 _p(b1), _p(ws.h), _p(ws.hmax), m, hidden, k, hidden, *_gemm_ws(dev), st)
-            call("mxq_quantize_int8_rowwise_absmax", _p(ws.h), _p(ws.hmax), _p(ws.hq), _p(ws.hs), m,
-                 hidden, st)
-        call("mxq_int8_gemm_dequant", _p(ws.hq), _p(w2), _p(ws.hs), _p(s2), s2.numel(), _p(b2),
-             _p(out), m, n, hidden, n, _lib.DTYPE_BF16, *_gemm_ws(dev, m, n, hidden), st)
+    _launch(dev, "mxq_quantize_int8_rowwise", _ptr(x2), _OUT_CODES[x.dtype], _ptr(ws.xq), _ptr(ws.xs), m, k,
+            _lib.ACT_NONE)
+    if hidden <= _GELU_QUANT_MAX_COLS:
+        _launch(dev, "mxq_int8_gemm_dequant", _ptr(ws.xq), _ptr(w1), _ptr(ws.xs), _ptr(s1), s1.numel(), _ptr(b1),
+                _ptr(ws.h), m, hidden, k, hidden, _lib.DTYPE_BF16, *_gemm_ws(dev, m, hidden, k))
+        _launch(dev, "mxq_quantize_int8_rowwise_gelu", _ptr(ws.h), _ptr(ws.h) if return_hidden else None,
+                _ptr(ws.hq), _ptr(ws.hs), m, hidden)
+    else:
+        _launch(dev, "mxq_fill_f32", _ptr(ws.hmax), 0.0, m)
+        _launch(dev, "mxq_int8_gemm_dequant_gelu_absmax", _ptr(ws.xq), _ptr(w1), _ptr(ws.xs), _ptr(s1), s1.numel(),
+                _ptr(b1), _ptr(ws.h), _ptr(ws.hmax), m, hidden, k, hidden, *_gemm_ws(dev))
+        _launch(dev, "mxq_quantize_int8_rowwise_absmax", _ptr(ws.h), _ptr(ws.hmax), _ptr(ws.hq), _ptr(ws.hs), m,
+                hidden)
+    _launch(dev, "mxq_int8_gemm_dequant", _ptr(ws.hq), _ptr(w2), _ptr(ws.hs), _ptr(s2), s2.numel(), _ptr(b2),
+            _ptr(out), m, n, hidden, n, _lib.DTYPE_BF16, *_gemm_ws(dev, m, n, hidden))
     out = out.reshape(*x.shape[:-1], n)
     return (out, ws.h.reshape(*x.shape[:-1], hidden)) if return_hidden else out
 
@@ -778,7 +812,7 @@ def int8_linear_gated_residual_(residual: torch.Tensor, x: torch.Tensor, weight:
         gate = gate.reshape(1, -1)
     if gate.dim() != 2 or gate.shape[1] != n:
         raise ValueError(f"gate must be [rows, {n}], got {tuple(gate.shape)}")
-    g = gate.to(device=dev, dtype=torch.bfloat16).contiguous()
+    g = _vector(gate, torch.bfloat16, dev)
     if isinstance(gate_rows, torch.Tensor):
         gr = _row_map(gate_rows, rows, g.shape[0], dev, "gate_rows", "gate_rows index outside the gate")
     else:
@@ -795,7 +829,7 @@ def int8_linear_gated_residual_(residual: torch.Tensor, x: torch.Tensor, weight:
         raise ValueError(f"Input and weight inner dimensions must match, got {width} and {weight.shape[-1]}")
     if act and x.dtype == torch.float32:
         raise NotImplementedError(f"input_act={input_act!r} needs a bfloat16 or float16 input")
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     if convrot:
         _check_power_of_four(convrot_groupsize)
         if width % convrot_groupsize:
@@ -804,9 +838,8 @@ def int8_linear_gated_residual_(residual: torch.Tensor, x: torch.Tensor, weight:
     else:
         q, xs = quantize_int8_rowwise(x2, input_act=input_act)
     q2, w2, k = _pad_k(q, weight)
-    with torch.cuda.device(dev):
-        call("mxq_int8_gemm_gated_residual", _p(q2), _p(w2), _p(xs), _p(ws), ws.numel(), _p(b), _p(res2),
-             res2.stride(0), _p(g), g.stride(0), g.shape[0], _p(gr), rows, n, k, *_gemm_ws(dev, rows, n, k), _stream(dev))
+    _launch(dev, "mxq_int8_gemm_gated_residual", _ptr(q2), _ptr(w2), _ptr(xs), _ptr(ws), ws.numel(), _ptr(b), _ptr(res2),
+            res2.stride(0), _ptr(g), g.stride(0), g.shape[0], _ptr(gr), rows, n, k, *_gemm_ws(dev, rows, n, k))
     return residual
 
 
@@ -854,7 +887,7 @@ def prepare_swiglu_fc1(qweight: torch.Tensor, weight_scale: torch.Tensor,
         raise NotImplementedError("the SwiGLU epilogue needs 2 x inner to be a multiple of 32")
     dev = qweight.device
     order = _swiglu_order(n2, dev)
-    ws = _weight_scale(weight_scale, n2, dev)
+    ws = _weight_scale(weight_scale, n2, dev).reshape(-1)
     ws = ws if ws.numel() == 1 else ws[order].contiguous()
     b = None if bias is None else bias.to(device=dev, dtype=torch.bfloat16).reshape(-1)[order].contiguous()
     return PreparedSwiGLUFc1(qweight[order].contiguous(), ws, b, n2 // 2)
@@ -870,7 +903,7 @@ def int8_swiglu_fc1(x_qdata: torch.Tensor, x_scale: torch.Tensor, fc1: PreparedS
         raise ValueError("Input and weight inner dimensions must match")
     dev = _require_gpu(x_qdata, fc1.qweight)
     m, n2 = x_qdata.shape[0], fc1.qweight.shape[0]
-    xs = x_scale.to(device=dev, dtype=torch.float32).reshape(-1).contiguous()
+    xs = _vector(x_scale, torch.float32, dev)
     if xs.numel() != m:
         raise ValueError(f"x_scale has {xs.numel()} entries, expected {m}")
     if out is None:
@@ -884,9 +917,8 @@ def int8_swiglu_fc1(x_qdata: torch.Tensor, x_scale: torch.Tensor, fc1: PreparedS
     if m == 0:
         return h
     q2, w2, k = _pad_k(x_qdata.contiguous(), fc1.qweight)
-    with torch.cuda.device(dev):
-        call("mxq_int8_gemm_dequant_swiglu", _p(q2), _p(w2), _p(xs), _p(fc1.scale), fc1.scale.numel(),
-             _p(fc1.bias), _p(h), m, n2, k, h.stride(0), *_gemm_ws(dev, m, n2, k, 2), _stream(dev))
+    _launch(dev, "mxq_int8_gemm_dequant_swiglu", _ptr(q2), _ptr(w2), _ptr(xs), _ptr(fc1.scale), fc1.scale.numel(),
+            _ptr(fc1.bias), _ptr(h), m, n2, k, h.stride(0), *_gemm_ws(dev, m, n2, k, 2))
     return h
 
 
@@ -920,7 +952,7 @@ def h3_mlp_(residual: torch.Tensor, norm, shift: torch.Tensor, scale: torch.Tens
 
 def _srel_code(s_rel: torch.Tensor) -> tuple[torch.Tensor, int]:
     if s_rel.dtype == torch.float8_e4m3fn:
-        return s_rel.contiguous().view(torch.uint8), _lib.DTYPE_E4M3
+        return s_rel.contiguous(), _lib.DTYPE_E4M3
     return s_rel.to(torch.float32).contiguous(), _lib.DTYPE_F32
 
 
@@ -1002,27 +1034,28 @@ def w4a8_int8_linear(x: torch.Tensor, qdata: torch.Tensor, s_rel: torch.Tensor, 
     if convrot_groupsize:
         if k % convrot_groupsize:
             raise ValueError(f"ConvRot group size {convrot_groupsize} does not divide input features {k}")
-        xq, xs = quantize_int8_rowwise_convrot(x.reshape(-1, k), convrot_groupsize)
+        xq, xs = quantize_int8_rowwise_convrot(x if x.dim() == 2 else x.reshape(-1, k), convrot_groupsize)
     else:
-        xq, xs = quantize_int8_rowwise(x.reshape(-1, k))
+        xq, xs = quantize_int8_rowwise(x if x.dim() == 2 else x.reshape(-1, k))
     m = xq.shape[0]
     out = torch.empty((m, n), dtype=out_dtype, device=dev)
     if m == 0:
         return out.reshape(*lead, n)
     sr, scode = _srel_code(s_rel.to(dev))
-    cb = None if codebook is None else codebook.to(device=dev, dtype=torch.float32).contiguous()
-    sch = s_channel.to(device=dev, dtype=torch.float32).contiguous()
+    cb = None if codebook is None else _vector(codebook, torch.float32, dev)
+    sch = _vector(s_channel, torch.float32, dev)
     b = _bias(bias, n, out_dtype, dev)
+    qd = qdata.contiguous()
     chunk = w4a8_decode_chunk(n, k)
     work = torch.empty((chunk, k), dtype=torch.int8, device=dev)
-    with torch.cuda.device(dev):
-        call("mxq_w4a8_codebook_gemm", _p(xq), _p(qdata.contiguous()), _p(sr), scode, _p(cb), _p(sch),
-             _p(xs), _p(b), _p(work), _p(out), m, n, k, group_size, chunk, code, *_gemm_ws(dev, m, min(chunk, n), k), _stream(dev))
-        if correction is not None:
-            sx = torch.empty((m, k // group_size), dtype=out_dtype, device=dev)
-            call("mxq_int8_group_sums", _p(xq), _p(xs), _p(sx), m, k, group_size, code, _stream(dev))
+    _launch(dev, "mxq_w4a8_codebook_gemm", _ptr(xq), _ptr(qd), _ptr(sr), scode, _ptr(cb), _ptr(sch),
+            _ptr(xs), _ptr(b), _ptr(work), _ptr(out), m, n, k, group_size, chunk, code, *_gemm_ws(dev, m, min(chunk, n), k))
+    if correction is not None:
+        sx = torch.empty((m, k // group_size), dtype=out_dtype, device=dev)
+        _launch(dev, "mxq_int8_group_sums", _ptr(xq), _ptr(xs), _ptr(sx), m, k, group_size, code)
+        with torch.cuda.device(dev):
             out.addmm_(sx, correction.to(device=dev, dtype=out_dtype))
-    return out.reshape(*lead, n)
+    return out if x.dim() == 2 else out.reshape(*lead, n)
 
 
 class PreparedW4A8Grouped:
@@ -1081,24 +1114,23 @@ def w4a8_grouped_linear(x: torch.Tensor, qdata: torch.Tensor | PreparedW4A8Group
     if x.dtype == torch.int8:
         if x_scale is None:
             raise ValueError("an int8 input needs x_scale")
-        xq = x.reshape(-1, k).contiguous()
-        xs = x_scale.to(device=dev, dtype=torch.float32).reshape(-1).contiguous()
+        xq = _rows(x, k)
+        xs = _vector(x_scale, torch.float32, dev)
         if xs.numel() != xq.shape[0]:
             raise ValueError(f"x_scale has {xs.numel()} entries, expected {xq.shape[0]}")
     else:
-        xq, xs = quantize_int8_rowwise(x.reshape(-1, k))
+        xq, xs = quantize_int8_rowwise(x if x.dim() == 2 else x.reshape(-1, k))
     lead = x.shape[:-1]
     m = xq.shape[0]
     out = torch.empty((m, n), dtype=out_dtype, device=dev)
     if m == 0:
         return out.reshape(*lead, n)
-    gs = group_scale.to(device=dev, dtype=torch.float16).contiguous()
+    gs = _vector(group_scale, torch.float16, dev)
     b = _bias(bias, n, out_dtype, dev)
+    qd = qdata.contiguous()
     entry = "mxq_w4a8_gemm_grouped_prepared" if prepared else "mxq_w4a8_gemm_grouped"
-    with torch.cuda.device(dev):
-        call(entry, _p(xq), _p(xs), _p(qdata.contiguous()), _p(gs), _p(b), _p(out),
-             m, n, k, group_size, n, code, _stream(dev))
-    return out.reshape(*lead, n)
+    _launch(dev, entry, _ptr(xq), _ptr(xs), _ptr(qd), _ptr(gs), _ptr(b), _ptr(out), m, n, k, group_size, n, code)
+    return out if x.dim() == 2 else out.reshape(*lead, n)
 
 
 # ---------------------------------------------------------------------------------------
