@@ -44,6 +44,7 @@
 //               fused_mlp.py:157-219; y * gate is exact in fp32, so one fp32 add, then RNE).
 
 #include "act_rot.h"
+#include "w4a8_common.h"
 
 namespace mxq {
 
@@ -1596,6 +1597,25 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(GemmArgs p, const int
   } else {
     store_run<kElem>(p.d, p.ldd, row, col, nout, p.vec_store && col + 4 <= nout, w);
   }
+}
+
+int launch_split_dequant(const int32_t* part, int splits, int64_t ldp, const float* xs, const float* ws, const void* bias,
+                         void* d, int64_t M, int64_t N, int64_t ldd, int out_dtype, hipStream_t st) {
+  GemmArgs g{};
+  g.xs = xs; g.ws = ws; g.bias = bias; g.d = d; g.M = M; g.N = N; g.ldd = ldd;
+  g.ws_per_channel = 1;
+  g.splits = splits;
+  g.slice_stride = M * ldp * 4;
+  const int elem = out_dtype == MXQ_DTYPE_F32 ? 4 : 2;
+  g.vec_store = ((uintptr_t)d % (4 * elem) == 0) && (ldd % 4 == 0);
+  const unsigned grid = (unsigned)((M * ((N + 3) / 4) + 255) / 256);
+  switch (out_dtype) {
+    case MXQ_DTYPE_F32: split_reduce_kernel<kEpiDequant, 0><<<grid, 256, 0, st>>>(g, part, ldp); break;
+    case MXQ_DTYPE_F16: split_reduce_kernel<kEpiDequant, 1><<<grid, 256, 0, st>>>(g, part, ldp); break;
+    case MXQ_DTYPE_BF16: split_reduce_kernel<kEpiDequant, 2><<<grid, 256, 0, st>>>(g, part, ldp); break;
+    default: return mxq_set_error(MXQ_ERR_UNSUPPORTED, "output dtype code %d", out_dtype);
+  }
+  return mxq_check_launch("split_reduce_kernel");
 }
 
 template <int kEpi, int kOut>
