@@ -212,3 +212,34 @@ def test_convrot_nan_and_inf_rows_follow_the_oracle(dev, g):
         qr2, sr2, _ = cr.convrot_quantize_f32(xf.numpy(), g or 256)
     assert np.array_equal(q2.cpu().numpy(), qr2)
     assert np.array_equal(s2.cpu().numpy(), sr2, equal_nan=True)
+
+
+@pytest.mark.parametrize("k,g,act", [(256, 256, None), (3072, 256, None), (5376, 256, None), (6144, 64, "swiglu"),
+                                     (8448, 256, None), (14336, 256, "swiglu"), (16384, 16, "gelu_tanh"), (16640, 256, None),
+                                     (20480, 256, "gelu_tanh"), (20480, 0, None)])
+def test_convrot_row_splits_agree(dev, k, g, act):
+    """A row's values do not depend on how many rows the call has: both sides of each row count at which
+    the block layout changes, for widths of every layout, against one large call, whose first rows the oracle checks."""
+    x = torch.randn(1100, k * (2 if act == "swiglu" else 1), generator=gen(k + g)).to(torch.bfloat16)
+    xd = x.to(dev)
+    q, s = _mx().quantize_int8_rowwise_convrot(xd, g, act)
+    qr, sr, _ = cr.convrot_quantize_bf16(bits(x[:3]), g, act)
+    assert np.array_equal(q[:3].cpu().numpy(), qr) and np.array_equal(s[:3].cpu().numpy(), sr)
+    for m in (1, 2, 255, 256, 257, 512, 513, 1024, 1025):
+        print(f"convrot row splits k={k} g={g} {act} m={m}", flush=True)
+        qm, sm = _mx().quantize_int8_rowwise_convrot(xd[:m], g, act)
+        assert torch.equal(qm, q[:m]) and torch.equal(sm, s[:m])
+
+
+@pytest.mark.parametrize("k", [512, 5376, 8448, 16384])
+def test_rms_adaln_row_splits_agree(dev, k):
+    """The same behind the RMS adaLN front end, with and without the 1 + scale table (12288 rows)."""
+    x = torch.randn(12289, k, generator=gen(k)).to(torch.bfloat16).to(dev)
+    vec = [bf16_vec(k, i, 0.2).to(dev) for i in range(5)]
+    scale, shift = torch.stack(vec[:2]), torch.stack(vec[2:4])
+    call = lambda m: _mx().rms_adaln_quantize_int8(x[:m], (1 + vec[4], 1e-6), shift, scale, ((0, 1, 1), (1, m, 0)) if m > 1 else ((0, 1, 1),))
+    q, s = call(12289)
+    for m in (1, 256, 257, 512, 513, 1025, 12288):
+        print(f"rms row splits k={k} m={m}", flush=True)
+        qm, sm = call(m)
+        assert torch.equal(qm, q[:m]) and torch.equal(sm, s[:m])

@@ -296,12 +296,13 @@ int launch_convrot(const CrArgs& a, int nw, hipStream_t st) {
 // the float64 -> bfloat16 rounding done in pairs (the midpoint correction of f64_to_bf16_bits
 // runs only for a unit where some float32 value lands on a bfloat16 midpoint) and rows whose
 // absmax is finite quantized by the finite-row path.
-// A launch of at most 8 rows (one token's row: the M = 1 linear, decode) is bound by the latency
-// of one row's work, not by throughput: it takes the fewest units per group, one unit a group in
-// blocks of up to kUnitLatWaves waves (K = 5376: 21 groups in 6 waves; the kernel 5.4 -> 3.8 us,
-// near the ~3.4 us of an empty launch, against 3 units a group in 2 waves).
+// Few rows (one token's to some hundreds) are bound by the latency of one row's work, not by throughput: they take
+// a block per row and the fewest units per group for which all rows run at once (few_row_split). In us, against the
+// throughput split: 77 x 5376 7.0 -> 4.8, 77 x 7168 8.3 -> 4.8, 333 x 14336 SwiGLU 19.2 -> 16.1, 333 x 5376 with the RMS
+// front end 11.1 -> 8.6. Rows of 16640 to 20480 columns take five units a group (2048 x 20480 54.2 -> 40.8 against the window
+// form).
 constexpr int kUnitMaxWaves = 4;
-constexpr int kUnitLatWaves = 6;
+constexpr int kUnitRowWaves = 16;  // waves of a few-row block, at most (eight with the RMS front end's registers)
 
 // The rotation of one unit up to the transposed layout: digits 0 and 1 in the lane; for
 // kDigits >= 3 each 16-lane group transposes its 16 x 16 float64 values through its LDS region
@@ -371,7 +372,10 @@ __global__ __launch_bounds__(kWaves * 64) void convrot_units_kernel(CrArgs p, in
   constexpr double kInv = 1.0 / (double)(1 << kDigits);     // 1/sqrt(G), exact
   __shared__ uint32_t red_max[2][4 * kWaves];
   __shared__ double red_ss[2][4 * kWaves];
-  extern __shared__ __attribute__((aligned(16))) double tbuf[];  // kTWave per wave of the block
+  // kTWave per wave of the block; a few-row block's may exceed the 64 KB of dynamic LDS, so it is static
+  extern __shared__ __attribute__((aligned(16))) double tdyn[];
+  __shared__ __attribute__((aligned(16))) double tstat[kWaves > kUnitMaxWaves ? kWaves * kTWave : 1];
+  double* tbuf = kWaves > kUnitMaxWaves ? tstat : tdyn;
   const int wave = threadIdx.x >> 6;
   const int grp = threadIdx.x >> 4, gl = threadIdx.x & 15;
   const int slot = grp / gr, gi = grp - slot * gr;
@@ -566,7 +570,8 @@ struct UnitSplit {
 UnitSplit unit_split(int units) {
   UnitSplit best{0, 0, 0, 0};
   double best_util = -1.0;
-  for (int nu = 1; nu <= 4; ++nu) {
+  for (int nu = units > 4 * 4 * kUnitMaxWaves ? 5 : 1; nu <= 5; ++nu) {
+    if (nu == 5 && best.nu) break;  // five only where four would need larger blocks (K > 16384)
     const int gr = (units + nu - 1) / nu;
     if (gr > 4 * kUnitMaxWaves) continue;
     for (int rpb = 1; rpb * gr <= 4 * kUnitMaxWaves; ++rpb) {
@@ -581,6 +586,18 @@ UnitSplit unit_split(int units) {
   return best;
 }
 
+// A row per block and the fewest units per group for which every row's block is resident at once: one block of more
+// than eight waves per CU (156 KB of transpose buffers), two of five to eight, sixteen waves in smaller ones.
+UnitSplit few_row_split(int units, int64_t rows, bool mod) {
+  for (int nu = 1; nu <= 4; ++nu) {
+    const int gr = (units + nu - 1) / nu, waves = (gr + 3) / 4;
+    if (waves > (mod ? 8 : kUnitRowWaves) || (waves > kUnitMaxWaves && nu > 2)) continue;
+    const int per_cu = waves > 8 ? 1 : waves > kUnitMaxWaves ? 2 : 16 / waves;
+    if (rows <= (int64_t)std::min(mxq_cu_count(), 256) * per_cu) return UnitSplit{nu, gr, 1, waves};
+  }
+  return unit_split(units);
+}
+
 template <int kAct, int kMod, int kDigits, bool kTab = false>
 int launch_units(const CrArgs& a, const UnitSplit& u, hipStream_t st) {
   // One row batch per block (measured faster at 720p than persistent blocks that prefetch the
@@ -588,33 +605,35 @@ int launch_units(const CrArgs& a, const UnitSplit& u, hipStream_t st) {
   const unsigned grid = (unsigned)std::min<int64_t>((a.rows + u.rpb - 1) / u.rpb, 1 << 20);
   const unsigned threads = (unsigned)(u.waves * 64);
   const size_t lds = (size_t)u.waves * kTWave * sizeof(double);
-  if (u.waves > kUnitMaxWaves) {  // the few-row split: one unit a group
-    convrot_units_kernel<kAct, kMod, kDigits, 1, kTab, 1, kUnitLatWaves><<<grid, threads, lds, st>>>(a, u.gr, u.rpb);
+  if (u.waves > kUnitMaxWaves) {  // few_row_split: one or two units a group
+    if (u.waves <= 8) {
+      if (u.nu == 1)
+        convrot_units_kernel<kAct, kMod, kDigits, 1, kTab, 1, 8><<<grid, threads, 0, st>>>(a, u.gr, u.rpb);
+      else
+        convrot_units_kernel<kAct, kMod, kDigits, 2, kTab, 1, 8><<<grid, threads, 0, st>>>(a, u.gr, u.rpb);
+    } else if constexpr (kMod == kModNone) {
+      if (u.nu == 1)
+        convrot_units_kernel<kAct, kMod, kDigits, 1, kTab, 1, kUnitRowWaves><<<grid, threads, 0, st>>>(a, u.gr, u.rpb);
+      else
+        convrot_units_kernel<kAct, kMod, kDigits, 2, kTab, 1, kUnitRowWaves><<<grid, threads, 0, st>>>(a, u.gr, u.rpb);
+    }
     return mxq_check_launch("convrot_units_kernel");
   }
   switch (u.nu) {
     case 1: convrot_units_kernel<kAct, kMod, kDigits, 1, kTab><<<grid, threads, lds, st>>>(a, u.gr, u.rpb); break;
     case 2: convrot_units_kernel<kAct, kMod, kDigits, 2, kTab><<<grid, threads, lds, st>>>(a, u.gr, u.rpb); break;
     case 3: convrot_units_kernel<kAct, kMod, kDigits, 3, kTab><<<grid, threads, lds, st>>>(a, u.gr, u.rpb); break;
-    default: convrot_units_kernel<kAct, kMod, kDigits, 4, kTab><<<grid, threads, lds, st>>>(a, u.gr, u.rpb); break;
+    case 4: convrot_units_kernel<kAct, kMod, kDigits, 4, kTab><<<grid, threads, lds, st>>>(a, u.gr, u.rpb); break;
+    default:
+      if constexpr (kMod == kModNone)
+        convrot_units_kernel<kAct, kMod, kDigits, 5, kTab><<<grid, threads, lds, st>>>(a, u.gr, u.rpb);
   }
   return mxq_check_launch("convrot_units_kernel");
 }
 
 template <int kAct, int kMod, bool kTab = false>
 int launch_units_digits(const CrArgs& a, hipStream_t st) {
-  UnitSplit u = unit_split(a.K >> 8);
-  if (a.rows <= 8) {  // latency-bound: fewest units per group, one row a block
-    const int units = (int)(a.K >> 8);
-    if (units <= 4 * kUnitLatWaves) {
-      u = UnitSplit{1, units, 1, (units + 3) / 4};
-    } else {
-      for (int nu = 1; nu <= 4; ++nu) {
-        const int gr = (units + nu - 1) / nu;
-        if (gr <= 4 * kUnitMaxWaves) { u = UnitSplit{nu, gr, 1, (gr + 3) / 4}; break; }
-      }
-    }
-  }
+  const UnitSplit u = few_row_split((int)(a.K >> 8), a.rows, kMod != kModNone);
   switch (a.digits) {
     case 0: return launch_units<kAct, kMod, 0, kTab>(a, u, st);
     case 1: return launch_units<kAct, kMod, 1, kTab>(a, u, st);
@@ -624,8 +643,11 @@ int launch_units_digits(const CrArgs& a, hipStream_t st) {
   }
 }
 
-// The unit form takes bf16 rows with G <= 256 and K a multiple of 256 up to 4 * 32 units.
-bool units_fit(int64_t cols, int digits) { return digits <= 4 && cols % 256 == 0 && cols <= 256 * 4 * 4 * kUnitMaxWaves; }
+// The unit form takes bf16 rows with G <= 256 and K a multiple of 256, up to five units per group (four behind the
+// RMS front end).
+bool units_fit(int64_t cols, int digits, bool mod) {
+  return digits <= 4 && cols % 256 == 0 && cols <= 256 * (mod ? 4 : 5) * 4 * kUnitMaxWaves;
+}
 
 __global__ __launch_bounds__(256) void swiglu_kernel(const uint16_t* __restrict__ x, uint16_t* __restrict__ y,
                                                       int64_t rows, int64_t cols) {
@@ -635,6 +657,10 @@ __global__ __launch_bounds__(256) void swiglu_kernel(const uint16_t* __restrict_
     y[i] = (uint16_t)swiglu_bf16(x[r * 2 * cols + c], x[r * 2 * cols + cols + c]);
   }
 }
+
+// Rows past which forming the table is worth its launch (5376 columns, two rows of modulation: the table saves 3.0 us
+// of 69.8 at 8000 rows and 6.4 of 131.1 at 16000, its launch takes 4.7).
+constexpr int64_t kTabRows = 12288;
 
 // t[m, c] = bf16(1 + scale[m, c]) for the modulation rows (c < cols, row stride ld): the factor
 // every token of segment m multiplies its normalized value by, formed once per call instead of
@@ -694,7 +720,7 @@ extern "C" int mxq_quantize_int8_rowwise_convrot(const void* x, int x_dtype, int
       default: return launch_convrot<MXQ_ACT_SWIGLU, MXQ_DTYPE_F16, kModNone>(a, nw, st);
     }
   }
-  if (units_fit(cols, digits)) {
+  if (units_fit(cols, digits, false)) {
     switch (input_act) {
       case MXQ_ACT_NONE: return launch_units_digits<MXQ_ACT_NONE, kModNone>(a, st);
       case MXQ_ACT_GELU_TANH: return launch_units_digits<MXQ_ACT_GELU_TANH, kModNone>(a, st);
@@ -760,8 +786,8 @@ static int rms_adaln_launch(const void* x, const void* norm_weight, const void* 
     if (q) return launch_convrot<MXQ_ACT_NONE, MXQ_DTYPE_F16, kModQuant>(a, nw, st);
     return launch_convrot<MXQ_ACT_NONE, MXQ_DTYPE_F16, kModOnly>(a, nw, st);
   }
-  if (units_fit(cols, digits)) {
-    if (q && workspace && workspace_bytes >= mod_count * ld_mod * 2 && (uintptr_t)workspace % 16 == 0) {
+  if (units_fit(cols, digits, true)) {
+    if (q && rows > kTabRows && workspace && workspace_bytes >= mod_count * ld_mod * 2 && (uintptr_t)workspace % 16 == 0) {
       // bf16(1 + scale) of every modulation row into the workspace, then the kernel reads it there
       uint16_t* t = (uint16_t*)workspace;
       const int64_t n = mod_count * (cols / 8);
