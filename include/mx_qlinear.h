@@ -166,6 +166,16 @@ int mxq_int8_gemm_plan(int64_t M, int64_t N, int64_t K, int table_epilogue, int6
                        int64_t* plan);
 
 /*
+ * The tile-rows an M x N x K problem runs instead of that plan's, when it fills the CUs better (GEMMs of up to
+ * sixteen rounds of tiles and K >= 2048; the outputs are the same, bit for bit): plan[0] 0 if none, else the rows of
+ * its short tiles (192 or 128; 256: no short ones), plan[1] tile-rows of 256, plan[2] short tile-rows behind them,
+ * plan[3] 1 when the tiles are claimed from the workspace's counters. All tiles have 256 columns. plan holds
+ * 4 entries. A problem whose K is cut (mxq_int8_gemm_workspace) runs neither. Host only; no reference counterpart.
+ */
+int mxq_int8_gemm_short_plan(int64_t M, int64_t N, int64_t K, int table_epilogue, int64_t workspace_bytes,
+                             int64_t* plan);
+
+/*
  * Raw INT8 GEMM: C[m, n] = sum_k A[m, k] * B[n, k] in int32.
  *   a [M, K] int8 row-major; b [N, K] int8 row-major (the checkpoint's [out, in] layout);
  *   c [M, ldc] int32. K must be a multiple of 16.

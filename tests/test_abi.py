@@ -340,3 +340,26 @@ def test_bench_matches_kernel_instances_by_template_prefix():
     assert not m("gemm_i8_kernel<1, 2, 128>", "void mxq::gemm_i8_kernel<1, 2, 256, false>(mxq::GemmArgs)")
     assert not m("gemm_i8_kernel<1, 2, 256>", "void mxq::gemm_i8_kernel<4, 2, 256, false>(mxq::GemmArgs)")
     assert m("w4a8_g128_kernel", "void mxq::w4a8_g128_kernel<128, 3>(mxq::G128Args)")
+
+
+@pytest.mark.parametrize("n", [1, 255, 3072, 5120, 5377, 21504, 70000])
+@pytest.mark.parametrize("table", [0, 2])
+def test_short_tile_plan_covers_every_row(lib, n, table):
+    """256-row tile-rows and the short ones behind them hold every row and leave no tile-row empty; claimed plans
+    need the counters, and a problem of fewer tiles than CUs claims nothing."""
+    from mx_qlinear import _lib
+
+    seen = set()
+    for m in [1, 128, 129, 192, 193, 256, 257, *range(300, 9000, 237), 40000, 75600]:
+        for space in (0, 1152, _lib.GEMM_WORKSPACE_BYTES):
+            p = _lib.gemm_short_plan(m, n, 5120, table, space)
+            seen.add((p["rows"], p["queued"]))
+            if p["rows"] == 0:
+                continue
+            below = 256 * p["tiles_m"] + p["rows"] * (p["short_m"] - 1 if p["rows"] < 256 else 0)
+            assert (below - 256 if p["rows"] == 256 else below) < m <= 256 * p["tiles_m"] + p["rows"] * (p["rows"] < 256) * p["short_m"]
+            assert not p["queued"] or space >= 3072
+            # one tile each: only where no tile waits for another's workgroup to claim it
+            assert p["queued"] or p["rows"] == 256 or (p["tiles_m"] == 0 and p["short_m"] * -(-n // 256) <= 256)
+    assert n < 3072 or len(seen) > 1
+    assert _lib.gemm_short_plan(4097, 21504, 2032)["rows"] == 0  # short K keeps the uniform tiles

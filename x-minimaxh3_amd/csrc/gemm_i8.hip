@@ -62,18 +62,22 @@ constexpr int kGemmThreads = 256;                       // 4 waves as 2 x 2
 // A B chunk is then 12 KB in a 16 KB slot, and the ring carries 28 KB per stage instead of 32.
 // kTM = 64, 32: 64 or 32 rows of the same deep ring, the four waves side by side along the columns, for
 // the K slices of problems of that few rows (split_plan).
+// kPP with kTM = 192, 128: 192 or 128 rows of the ping-pong tile (waves of 96 x 64 or 64 x 64), for the rows that
+// whole 256-row tiles would leave to a mostly empty last round (short_plan). Its A chunks fill part of a slot.
 template <int kT, bool kDeep = false, bool kPP = false, int kTN = kT, int kTM = kT>
 struct TileCfg {
   static_assert(kT == 128 || !kDeep, "the deep ring exists for 128-tiles only");
   static_assert(kT == 256 || !kPP, "the ping-pong schedule exists for 256-tiles only");
   static_assert(kTN == kT || (kDeep && kTN == 96), "128 x 96 tiles run the deep ring only");
-  static_assert(kTM == kT || (kDeep && kTN == kT && (kTM == 64 || kTM == 32)), "few-row tiles run the deep ring only");
+  static_assert(kTM == kT || (kDeep && kTN == kT && (kTM == 64 || kTM == 32)) ||
+                    (kPP && kTN == kT && (kTM == 192 || kTM == 128)),
+                "few-row tiles run the deep ring or the ping-pong schedule only");
   static constexpr bool kPingPong = kPP;
   static constexpr int kWaves = kPP ? 8 : 4;                    // two per SIMD with kPP
   static constexpr int kThreads = kWaves * 64;
   static constexpr int kBM = kTM, kBN = kTN;
   static constexpr int kWavesN = kPP || kTM < kT ? 4 : (kTN == kT ? 2 : 1);  // waves across the tile's columns
-  static constexpr int kWaveM = kPP ? kT / 2 : kTM / (kWaves / kWavesN), kWaveN = kTN / kWavesN;
+  static constexpr int kWaveM = kPP ? kTM / 2 : kTM / (kWaves / kWavesN), kWaveN = kTN / kWavesN;
   static constexpr int kBI = kWaveM / 32, kBJ = kWaveN / 32;
   static constexpr int kSlotBytes = kT * kBK;                  // one operand chunk of a stage (slot size)
   static constexpr int kLoads = kTM * kBK / 1024 / kWaves;      // direct-to-LDS loads per wave per A slot
@@ -131,6 +135,9 @@ struct GemmArgs {
   // Ping-pong kernel only: wg_per_xcd workgroups per XCD loop over the tiles, claiming them from
   // the counters (pp_tiles); n_claim is then the grid.
   int persistent;
+  // Short tiles (short_plan): short_m tile-rows of fewer rows from row short_first on, behind the tiles_m of 256.
+  int short_m;
+  int64_t short_first;
   // Split K (kEpiSplit): `splits` slices of slice_k K-bytes each (a multiple of kBK), slice s writing its int32 sums
   // at d + s * slice_stride.
   int splits;
@@ -613,7 +620,7 @@ MXQ_DEVICE void pp_frags(int lane, uint32_t slot_a, uint32_t slot_b, int wrow, i
 // B slot) follows each of the first kLoadsB MFMAs when `on`.
 template <class C, int kLoadsB, bool kCheck>
 MXQ_DEVICE void pp_mma(const v4i (&fa)[2][C::kBI], const v4i (&fb)[2][C::kBJ], v16i (&acc)[C::kBI][C::kBJ],
-                       const Loader<C::kLoads>& L, char* slot, int64_t k0, int64_t K, bool on) {
+                       const Loader<C::kLoads, C::kLoadsB>& L, char* slot, int64_t k0, int64_t K, bool on) {
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
@@ -624,11 +631,11 @@ MXQ_DEVICE void pp_mma(const v4i (&fa)[2][C::kBI], const v4i (&fb)[2][C::kBJ], v
     }
 }
 
-template <bool kB, bool kCheck, int kL>
-MXQ_DEVICE void pp_issue(const Loader<kL>& L, char* slot, int64_t k0, int64_t K, bool on) {
+template <bool kB, bool kCheck, int kL, int kLB>
+MXQ_DEVICE void pp_issue(const Loader<kL, kLB>& L, char* slot, int64_t k0, int64_t K, bool on) {
   if (on) {
 #pragma unroll
-    for (int t = 0; t < kL; ++t) issue_one<kB, kCheck>(L, slot, k0, K, t);
+    for (int t = 0; t < (kB ? kLB : kL); ++t) issue_one<kB, kCheck>(L, slot, k0, K, t);
   }
 }
 
@@ -645,7 +652,7 @@ MXQ_DEVICE void pp_barrier() {
 // latency then hides behind those iterations' MFMAs).
 template <class C, int kG, class BeforeTail>
 MXQ_DEVICE void pp_loop(const GemmArgs& p, char* lds, v16i (&acc)[C::kBI][C::kBJ], int wrow, int wcol,
-                        const Loader<C::kLoads>& ld, BeforeTail&& before_tail) {
+                        const Loader<C::kLoads, C::kLoadsB>& ld, BeforeTail&& before_tail) {
   constexpr int kSlotBytes = C::kSlotBytes, kSlots = C::kSlots, kL = C::kLoads;
   const int ktiles = (int)((p.K + kBK - 1) / kBK);
   const uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr_t)lds;
@@ -658,7 +665,7 @@ MXQ_DEVICE void pp_loop(const GemmArgs& p, char* lds, v16i (&acc)[C::kBI][C::kBJ
   pp_barrier();
   pp_issue<true, true>(ld, lds + 3 * kSlotBytes, kBK, p.K, ktiles > 1);
   if (ktiles > 1)
-    wait_vmcnt<kL>();
+    wait_vmcnt<C::kLoadsB>();
   else
     wait_vmcnt<0>();
   pp_barrier();
@@ -711,7 +718,7 @@ MXQ_DEVICE void pp_loop(const GemmArgs& p, char* lds, v16i (&acc)[C::kBI][C::kBJ
       pp_issue<true, !kSteady>(ld, slot_sa, k2, p.K, more2);
       wait_lgkm<0>();
     } else {
-      pp_mma<C, kL, !kSteady>(fa, fb, acc, ld, slot_sa, k2, p.K, more2);                 // P3
+      pp_mma<C, C::kLoadsB, !kSteady>(fa, fb, acc, ld, slot_sa, k2, p.K, more2);                 // P3
     }
     pp_barrier();
     (void)more1;
@@ -729,7 +736,7 @@ MXQ_DEVICE void pp_loop(const GemmArgs& p, char* lds, v16i (&acc)[C::kBI][C::kBJ
 
 // A tile's first operand chunks: A_0, B_0 and (when K has a second stage) A_1 into slots 0-2.
 template <class C>
-MXQ_DEVICE void pp_first_loads(const GemmArgs& p, char* lds, const Loader<C::kLoads>& ld) {
+MXQ_DEVICE void pp_first_loads(const GemmArgs& p, char* lds, const Loader<C::kLoads, C::kLoadsB>& ld) {
   pp_issue<false, true>(ld, lds, 0, p.K, true);
   pp_issue<true, true>(ld, lds + C::kSlotBytes, 0, p.K, true);
   pp_issue<false, true>(ld, lds + 2 * C::kSlotBytes, kBK, p.K, p.K > kBK);
@@ -737,7 +744,7 @@ MXQ_DEVICE void pp_first_loads(const GemmArgs& p, char* lds, const Loader<C::kLo
 
 // One of those three chunks: A_0 (part 0), B_0 (1), A_1 (2).
 template <class C>
-MXQ_DEVICE void pp_first_load_part(const GemmArgs& p, char* lds, const Loader<C::kLoads>& ld, int part) {
+MXQ_DEVICE void pp_first_load_part(const GemmArgs& p, char* lds, const Loader<C::kLoads, C::kLoadsB>& ld, int part) {
   if (part == 0) pp_issue<false, true>(ld, lds, 0, p.K, true);
   if (part == 1) pp_issue<true, true>(ld, lds + C::kSlotBytes, 0, p.K, true);
   if (part == 2) pp_issue<false, true>(ld, lds + 2 * C::kSlotBytes, kBK, p.K, p.K > kBK);
@@ -898,6 +905,8 @@ MXQ_DEVICE void gemm_epilogue(const GemmArgs& p, char* lds, v16i (&acc)[C::kBI][
       if constexpr (kEpi != kEpiGatedRes && jp == 0 && i < 3) {
         __builtin_amdgcn_sched_barrier(0);
         pre(i);
+        if constexpr (kBI < 3 && i == kBI - 1)  // too few block rows: the last one issues what is left
+          for (int part = kBI; part < 3; ++part) pre(part);
         __builtin_amdgcn_sched_barrier(0);
       }
       constexpr int kWords = kElem == 4 ? 4 : 2;
@@ -1011,12 +1020,10 @@ MXQ_DEVICE void gemm_epilogue(const GemmArgs& p, char* lds, v16i (&acc)[C::kBI][
   if constexpr (kEpi == kEpiSwiGLU) {
     // Every wave's kilobyte of the SiLU table has landed: only the `pre_loads` loads of the next
     // tile, issued after it, may stay in flight (a wait for more than those is still correct).
-    if (pre_loads >= 3 * C::kLoads)
-      wait_vmcnt<3 * C::kLoads>();
-    else if (pre_loads >= 2 * C::kLoads)
-      wait_vmcnt<2 * C::kLoads>();
-    else if (pre_loads >= C::kLoads)
-      wait_vmcnt<C::kLoads>();
+    if (pre_loads >= 2 * C::kLoads + C::kLoadsB)
+      wait_vmcnt<2 * C::kLoads + C::kLoadsB>();
+    else if (pre_loads >= C::kLoads + C::kLoadsB)
+      wait_vmcnt<C::kLoads + C::kLoadsB>();
     else
       wait_vmcnt<0>();
     barrier_no_drain();
@@ -1094,43 +1101,63 @@ MXQ_DEVICE void gemm_epilogue(const GemmArgs& p, char* lds, v16i (&acc)[C::kBI][
 // so the claim state costs no vector registers) and passes it to the workgroup through LDS. A
 // workgroup that finds every counter drained counts itself out (acquire-release); the last one
 // of the launch resets the counters for the next.
+//
+// Short tiles (kShort): the tile-rows behind the 256-row ones, all of them claimed, from counters of their own.
+constexpr int kShortCounters = 16 * 32;  // their place in the workspace, in words
+template <bool kShort>
 MXQ_DEVICE int pp_claim(const GemmArgs& p, int num, int& j) {
   const int x = blockIdx.x & 7;
   const bool lane0 = (tid_x() & 63) == 0;
   for (; j < 8; ++j) {
     const int y = (x + j) & 7;
     unsigned i = 0;
-    if (lane0) i = __hip_atomic_fetch_add(p.counters + y * 32, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (lane0)
+      i = __hip_atomic_fetch_add(p.counters + (kShort ? kShortCounters : 0) + y * 32, 1u, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
     i = (unsigned)__builtin_amdgcn_readfirstlane((int)i);
-    if (i < (unsigned)p.pool) {
-      int ys, yc;
-      xcd_range(y, num, ys, yc);
-      return ys + yc - p.pool + (int)i;
-    }
+    int ys, yc;
+    xcd_range(y, num, ys, yc);
+    const int pool = kShort ? yc : p.pool;
+    if (i < (unsigned)pool) return ys + yc - pool + (int)i;
   }
-  // Release: this workgroup's claims are ordered before its count; acquire: the last one sees
-  // every claim of the launch (the counts form one release sequence) before it resets.
-  if (lane0) {
+  return -1;
+}
+
+// A workgroup that has claimed its last tile counts itself out.
+// Release: this workgroup's claims are ordered before its count; acquire: the last one sees
+// every claim of the launch (the counts form one release sequence) before it resets.
+template <bool kShort>
+MXQ_DEVICE void pp_count_out(const GemmArgs& p) {
+  if ((tid_x() & 63) == 0) {
     const unsigned done = __hip_atomic_fetch_add(p.counters + 8 * 32, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
     if (done == (unsigned)p.n_claim - 1) {
-      for (int y = 0; y < 8; ++y) __hip_atomic_exchange(p.counters + y * 32, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (int y = 0; y < 8; ++y) {
+        __hip_atomic_exchange(p.counters + y * 32, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if constexpr (kShort)
+          __hip_atomic_exchange(p.counters + kShortCounters + y * 32, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
       __hip_atomic_exchange(p.counters + 8 * 32, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
-  return -1;
 }
 
 // The ping-pong kernel: its tiles (one, or a sequence when p.persistent), each through the main
 // loop and the epilogue. LDS at tile boundaries: slots 0-2 take the next tile's first chunks while
 // the epilogue keeps its per-column factors in slot 3 and its output staging in slot 4; the next
 // position passes from wave 0 to the workgroup through a word of slot 3.
-template <class C, int kEpi, int kOut>
+// kPart: all the tiles, the 256-row tiles ahead of short ones (the workgroup goes on with those), or the
+// short ones.
+enum { kPpAll = 0, kPpBig = 1, kPpShort = 2 };
+template <class C, int kEpi, int kOut, int kPart>
 MXQ_DEVICE void pp_tiles(const GemmArgs& p, char* lds) {
-  static_assert(C::kWaves == 8 && C::kSlots == 5 && C::kLoads == 4, "the ping-pong ring");
+  static_assert(C::kWaves == 8 && C::kSlots == 5 && C::kLoadsB == 4, "the ping-pong ring");
+  constexpr bool kShort = kPart == kPpShort;
   constexpr int kSlotBytes = C::kSlotBytes, kFactorBase = 3 * kSlotBytes, kStageBase = 4 * kSlotBytes;
   static_assert(kFactorBase + 2 * C::kBN * 4 + 4 <= kStageBase, "slot 3 holds the factors and the next position");
   const uint32_t next_word = lds_addr(lds + kFactorBase + 2 * C::kBN * 4);
-  const int num = p.tiles_m * p.tiles_n;
+  const int tiles_m = kShort ? p.short_m : p.tiles_m;
+  const int64_t m_first = kShort ? p.short_first : 0;
+  const int num = tiles_m * p.tiles_n;
   const bool wave0 = __builtin_amdgcn_readfirstlane(tid_x() >> 6) == 0;
   // Wave 0's next position: the next static one while there is one, then claims; -1 at the end.
   int static_next = -1, static_end = 0, claim_j = 0;
@@ -1142,15 +1169,21 @@ MXQ_DEVICE void pp_tiles(const GemmArgs& p, char* lds) {
       return pos;
     }
     static_next = -1;
-    return pp_claim(p, num, claim_j);
+    const int pos = pp_claim<kShort>(p, num, claim_j);
+    if (kPart != kPpBig && pos < 0) pp_count_out<kShort>(p);
+    return pos;
   };
   int pos;
   if (p.persistent) {
-    int s, c;
-    xcd_range(blockIdx.x & 7, num, s, c);
-    static_next = s + (int)(blockIdx.x >> 3);
-    static_end = s + c - p.pool;
-    if (static_next < static_end) {
+    if constexpr (kShort) {
+      pp_barrier();  // every wave has read the word that the first claim overwrites
+    } else {
+      int s, c;
+      xcd_range(blockIdx.x & 7, num, s, c);
+      static_next = s + (int)(blockIdx.x >> 3);
+      static_end = s + c - p.pool;
+    }
+    if (!kShort && static_next < static_end) {
       pos = static_next;
       static_next += p.wg_per_xcd;
     } else {  // more workgroups than static positions: the first tile is claimed too
@@ -1167,6 +1200,8 @@ MXQ_DEVICE void pp_tiles(const GemmArgs& p, char* lds) {
       pp_barrier();  // read before the first loads land in slot 3's neighbourhood
       if (pos < 0) return;
     }
+  } else if constexpr (kShort) {
+    pos = static_position(blockIdx.x, num);
   } else {
     pos = pick_tile(p, num, lds);
     if (pos < 0) return;
@@ -1178,17 +1213,17 @@ MXQ_DEVICE void pp_tiles(const GemmArgs& p, char* lds) {
   const int wcol = (wave & 1) * 128 + (wave >> 2) * 64;
   const bool group0 = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8)) == 0;
   int tm, tn;
-  tile_walk(pos, p.tiles_m, p.tiles_n, p.group_m, tm, tn);
-  int64_t m0 = (int64_t)tm * C::kBM, n0 = (int64_t)tn * C::kBN;
+  tile_walk(pos, tiles_m, p.tiles_n, p.group_m, tm, tn);
+  int64_t m0 = m_first + (int64_t)tm * C::kBM, n0 = (int64_t)tn * C::kBN;
   {
-    Loader<C::kLoads> first;
+    Loader<C::kLoads, C::kLoadsB> first;
     make_loader(first, p, m0, n0);
     pp_first_loads<C>(p, lds, first);
   }
   for (;;) {
     // (formed again per tile: the next tile's first loads use a copy of their own, so no loader
     // stays live through the epilogue)
-    Loader<C::kLoads> ld;
+    Loader<C::kLoads, C::kLoadsB> ld;
     make_loader(ld, p, m0, n0);
     v16i acc[C::kBI][C::kBJ];
 #pragma unroll
@@ -1218,19 +1253,19 @@ MXQ_DEVICE void pp_tiles(const GemmArgs& p, char* lds) {
       if (next >= 0) {
         if (part <= 0) {  // the first call
           int ntm, ntn;
-          tile_walk(next, p.tiles_m, p.tiles_n, p.group_m, ntm, ntn);
-          nm0 = (int64_t)ntm * C::kBM;
+          tile_walk(next, tiles_m, p.tiles_n, p.group_m, ntm, ntn);
+          nm0 = m_first + (int64_t)ntm * C::kBM;
           nn0 = (int64_t)ntn * C::kBN;
         }
         // (a loader formed per part: one kept live through the epilogue would take registers)
-        Loader<C::kLoads> next_ld;
+        Loader<C::kLoads, C::kLoadsB> next_ld;
         make_loader(next_ld, p, nm0, nn0);
         if (part < 0)
           pp_first_loads<C>(p, lds, next_ld);
         else
           pp_first_load_part<C>(p, lds, next_ld, part);
       }
-    }, next >= 0 ? (p.K > kBK ? 3 : 2) * C::kLoads : 0);
+    }, next >= 0 ? (p.K > kBK ? 2 : 1) * C::kLoads + C::kLoadsB : 0);
     if (next < 0) break;
     m0 = nm0;
     n0 = nn0;
@@ -1396,9 +1431,12 @@ __global__ __launch_bounds__((TileCfg<kT, kDeep, kPP, kTN, kTM>::kThreads), (Til
   typedef TileCfg<kT, kDeep, kPP, kTN, kTM> C;
   static_assert(kT == 256 || (kEpi != kEpiGelu && kEpi != kEpiSwiGLU), "table epilogues need the 160 KB ring");
   __shared__ __attribute__((aligned(16))) char lds[C::kLds];
-  if constexpr (kPP)
-    pp_tiles<C, kEpi, kOut>(p, lds);
-  else
+  if constexpr (kPP && kTM == kT) {
+    pp_tiles<C, kEpi, kOut, kPpAll>(p, lds);
+  } else if constexpr (kPP) {
+    if (p.tiles_m) pp_tiles<TileCfg<kT, kDeep, kPP>, kEpi, kOut, kPpBig>(p, lds);
+    pp_tiles<C, kEpi, kOut, kPpShort>(p, lds);
+  } else
     four_wave_tile<C, kEpi, kOut>(p, lds);
 }
 
@@ -1421,6 +1459,7 @@ struct GemmPlan {
   bool persistent;  // ping-pong workgroups that loop over their XCD's tiles (pp_tiles)
 };
 
+// The plan of uniform tiles (short_plan below replaces it where it fills the CUs better).
 // Problems with fewer 256-tiles than CUs run 128-tiles (four times as many workgroups). Larger ones
 // run 128-tiles too when their rounds finish first: 256 CUs hold 256 workgroups of 256-tiles or 512
 // of 128-tiles, and a round of 128-tiles takes about 0.55 of a round of 256-tiles (measured at
@@ -1477,6 +1516,72 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int table, int64_t workspace_byt
     }
   }
   return g;
+}
+
+// ---- short tiles ----
+// A GEMM of a few rounds of tiles loses the part of its last round that is empty: 4097 x 21504 is 1428 tiles of
+// 256 rows, 5.6 rounds on 256 CUs that take the time of six. Its last tile-rows then run as ping-pong tiles of 192 or 128
+// rows, which the workgroups claim once the 256-row tiles are done, and problems of less than a round may run
+// short tiles only. The rule compares the time the tiles take on the CUs, in hundredths of a round of
+// 256-tiles: a 192-row tile 90, a 128-row one 68 (their stages carry the same weight panel for fewer MFMAs); a
+// round of two 128 x 128 tiles per CU 70, of one 45. Fitted to 100 shapes of K = 3072 to 20480, N = 3072 to
+// 28672 and M = 140 to 9000, it picks within 0.4 % of the fastest on average and is 7 % faster than 256- and
+// 128-tiles alone. us before and after: 4331 x 5120 x 5120 134 -> 118, 2587 x 5376 x 14336 219 -> 179 (256-row tiles in
+// place of 128 x 128 ones), 3155 x 21504 x 5376 407 -> 331, 7512 x 5120 x 20480 791 -> 662, 333 x 28672 x 5376
+// SwiGLU 80 -> 72. K below 2048 and more than 16 rounds keep the plan above (an empty part of one round in
+// sixteen is 3 % at most); so do deep-ring problems, whose tiles all run at once.
+struct ShortPlan {
+  int rows;        // rows of a short tile: 192 or 128; 256: whole 256-tiles in place of 128-tiles; 0: plan_gemm's
+  int tiles_m;     // 256-row tile-rows
+  int short_m;     // short tile-rows, behind them
+  bool queued;     // looping workgroups that claim tiles (counters), else one tile each
+};
+constexpr int kShortQueueBytes = (kShortCounters + 8 * 32) * 4;
+static_assert(MXQ_GEMM_WORKSPACE_BYTES >= kShortQueueBytes, "workspace holds the short tiles' counters");
+
+// The time of `big` 256-tiles and then `shorts` tiles of cost c on `cus` CUs, each CU taking the next tile when
+// it is free.
+static int64_t tile_span(int64_t big, int64_t shorts, int c, int64_t cus) {
+  const int64_t q = big / cus * 100, late = big % cus;  // `late` CUs have one 256-tile more
+  int64_t end = late ? q + 100 : q, ta = q + c, tb = q + 100 + c;
+  while (shorts > 0) {
+    const bool first = !late || ta <= tb;
+    const int64_t t = first ? ta : tb;
+    shorts -= first ? cus - late : late;
+    (first ? ta : tb) += c;
+    end = std::max(end, t);
+  }
+  return end;
+}
+
+static ShortPlan short_plan(int64_t M, int64_t N, int64_t K, int table, const GemmPlan& g, int64_t workspace_bytes) {
+  ShortPlan best{};
+  const int64_t cus = std::max(1, mxq_cu_count()), tm = (M + 255) / 256, tn = (N + 255) / 256;
+  if (table == kTableGelu || g.deep || K < 2048 || tm > 16 * cus || tm * tn > 16 * cus) return best;
+  const bool counters = workspace_bytes >= kShortQueueBytes;
+  const int64_t whole = tile_span(tm * tn, 0, 100, cus);
+  int64_t least = whole;
+  if (g.tile == 128) {
+    const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n, rest = tiles % (2 * cus);
+    least = tiles / (2 * cus) * 70 + (rest > cus ? 70 : rest ? 45 : 0);
+    if (whole < least) {
+      least = whole;
+      best = ShortPlan{256, (int)tm, 0, counters && tm * tn > cus};
+    }
+  }
+  // (the last two rounds' tile-rows: shorter tiles further up gain nothing)
+  for (int h = 192; h >= 128; h -= 64)
+    for (int64_t r = tm - 1; r >= std::max<int64_t>(0, tm - 2 - 2 * cus / tn); --r) {
+      const int64_t rows = (M - 256 * r + h - 1) / h;
+      const bool queued = r > 0 || rows * tn > cus;
+      if (queued && !counters) continue;
+      const int64_t t = tile_span(r * tn, rows * tn, h == 192 ? 90 : 68, cus);
+      if (t + 2 < least) {  // (2: the change of tile height, so that ties keep whole tiles)
+        least = t + 2;
+        best = ShortPlan{h, (int)r, (int)rows, queued};
+      }
+    }
+  return best;
 }
 
 // ---- split K ----
@@ -1672,6 +1777,35 @@ static int launch_gemm(const GemmArgs& args0, void* workspace, int64_t workspace
     if (sp.splits && workspace && workspace_bytes >= MXQ_GEMM_WORKSPACE_BYTES + sp.bytes)
       return launch_split<kEpi, kOut>(args, sp, workspace, stream);
   }
+  if constexpr (kEpi != kEpiGelu) {
+    const ShortPlan sh = short_plan(args.M, args.N, args.K, kEpi == kEpiSwiGLU ? kTableSwiGLU : 0, g, workspace ? workspace_bytes : 0);
+    if (sh.rows) {
+      args.tiles_m = sh.tiles_m;
+      args.tiles_n = (int)((args.N + 255) / 256);
+      args.short_m = sh.short_m;
+      args.short_first = 256 * (int64_t)sh.tiles_m;
+      args.group_m = kGroupMPingPong;
+      args.persistent = sh.queued;
+      unsigned wgs = (unsigned)((sh.tiles_m + sh.short_m) * args.tiles_n);
+      args.pool = 0;
+      args.counters = nullptr;
+      if (sh.queued) {
+        args.pool = (int)(((int64_t)args.tiles_m * args.tiles_n / 8 + kPoolDiv - 1) / kPoolDiv);
+        args.wg_per_xcd = std::max(1, mxq_cu_count() / 8);
+        wgs = 8 * (unsigned)args.wg_per_xcd;
+        args.n_claim = (int)wgs;
+        args.counters = reinterpret_cast<unsigned*>(workspace);
+      }
+      constexpr unsigned kThreads = TileCfg<256, false, true>::kThreads;
+      if (sh.rows == 256)
+        gemm_i8_kernel<kEpi, kOut, 256, false, true><<<wgs, kThreads, 0, stream>>>(args);
+      else if (sh.rows == 192)
+        gemm_i8_kernel<kEpi, kOut, 256, false, true, 256, 192><<<wgs, kThreads, 0, stream>>>(args);
+      else
+        gemm_i8_kernel<kEpi, kOut, 256, false, true, 256, 128><<<wgs, kThreads, 0, stream>>>(args);
+      return mxq_check_launch("gemm_i8_kernel");
+    }
+  }
   const unsigned grid = (unsigned)g.grid;
   if constexpr (kEpi == kEpiSwiGLU) {
     // 256-tiles on the ping-pong schedule, the compact SiLU table in the epilogue
@@ -1726,8 +1860,23 @@ extern "C" int mxq_int8_gemm_workspace(int64_t M, int64_t N, int64_t K, int tabl
   const SplitPlan s = split_plan(M, N, K, table_epilogue);
   if (s.splits)
     *bytes = MXQ_GEMM_WORKSPACE_BYTES + s.bytes;
-  else if (plan_gemm(M, N, table_epilogue, MXQ_GEMM_WORKSPACE_BYTES).pool)
-    *bytes = MXQ_GEMM_WORKSPACE_BYTES;
+  else {
+    const GemmPlan g = plan_gemm(M, N, table_epilogue, MXQ_GEMM_WORKSPACE_BYTES);
+    const ShortPlan sh = short_plan(M, N, K, table_epilogue, g, MXQ_GEMM_WORKSPACE_BYTES);
+    if (sh.rows ? sh.queued : g.pool > 0) *bytes = MXQ_GEMM_WORKSPACE_BYTES;
+  }
+  return MXQ_OK;
+}
+
+extern "C" int mxq_int8_gemm_short_plan(int64_t M, int64_t N, int64_t K, int table_epilogue,
+                                        int64_t workspace_bytes, int64_t* plan) {
+  if (M <= 0 || N <= 0 || K <= 0 || !plan) return mxq_set_error(MXQ_ERR_INVALID, "GEMM plan needs a positive shape and an output");
+  if (table_epilogue < 0 || table_epilogue > kTableSwiGLU) return mxq_set_error(MXQ_ERR_INVALID, "table_epilogue must be 0, 1 or 2");
+  const ShortPlan sh = short_plan(M, N, K, table_epilogue, plan_gemm(M, N, table_epilogue, workspace_bytes), workspace_bytes);
+  plan[0] = sh.rows;
+  plan[1] = sh.tiles_m;
+  plan[2] = sh.short_m;
+  plan[3] = sh.queued;
   return MXQ_OK;
 }
 

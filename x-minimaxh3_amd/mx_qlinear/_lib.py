@@ -39,6 +39,7 @@ SIGNATURES: dict[str, list] = {
     "mxq_adaln": [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _F, _P],
     "mxq_adaln_quantize_int8": [_P, _P, _P, _I64, _I64, _F, _P, _P, _P, _I64, _I64, _P],
     "mxq_int8_gemm_plan": [_I64, _I64, _I64, _I, _I64, _P],
+    "mxq_int8_gemm_short_plan": [_I64, _I64, _I64, _I, _I64, _P],
     "mxq_int8_gemm_workspace": [_I64, _I64, _I64, _I, _P],
     "mxq_int8_gemm_i32": [_P, _P, _P, _I64, _I64, _I64, _I64, _P, _I64, _P],
     "mxq_int8_gemm_dequant": [_P, _P, _P, _P, _I64, _P, _P, _I64, _I64, _I64, _I64, _I, _P, _I64, _P],
@@ -112,6 +113,14 @@ def gemm_plan(m: int, n: int, k: int, table: int = 0, workspace_bytes: int = GEM
     call("mxq_int8_gemm_plan", m, n, k, int(table), workspace_bytes, out)
     return {"tile": out[0], "grid": out[1], "tiles": out[2], "pool": out[3], "wg_per_xcd": out[4],
             "ahead": out[5], "group_m": out[6], "persistent": bool(out[7]), "tile_n": out[8]}
+
+
+def gemm_short_plan(m: int, n: int, k: int, table: int = 0, workspace_bytes: int = GEMM_WORKSPACE_BYTES) -> dict:
+    """The tile-rows that replace gemm_plan's where they fill the CUs better (mxq_int8_gemm_short_plan):
+    rows of a short tile (0: gemm_plan holds), 256-row tile-rows, short tile-rows, whether tiles are claimed."""
+    out = (ctypes.c_int64 * 4)()
+    call("mxq_int8_gemm_short_plan", m, n, k, int(table), workspace_bytes, out)
+    return {"rows": out[0], "tiles_m": out[1], "short_m": out[2], "queued": bool(out[3])}
 
 
 @functools.lru_cache(maxsize=4096)
