@@ -317,3 +317,23 @@ def test_correction_through_the_module(dev):
                               spec=W4A8QuantSpec(group_size=g, convrot_groupsize=256), kernel=w4a8_kernel)
     want = _mx().w4a8_int8_linear(x, qd, s_rel, s_ch, correction=corr, bias=bias, group_size=g, convrot_groupsize=256)
     assert torch.equal(layer(x), want)
+
+
+# Few rows of group 128: workgroups of 32 columns whose eight waves take eight groups at once, with 32- or 64-row
+# tiles: group counts of one full round, a partial last round and several turns of the operand ring, ragged rows
+# and columns, both layouts, every output type.
+@pytest.mark.parametrize("m,n,k", [(1, 3000, 1024), (32, 136, 1152), (33, 264, 2176), (64, 4096, 1024), (31, 72, 6272),
+                                   (100, 3072, 1408), (80, 5120, 1152), (257, 136, 5248)])
+@pytest.mark.parametrize("prepared,out_dtype", [(True, torch.bfloat16), (False, torch.float16), (True, torch.float32)])
+def test_grouped_few_rows(dev, m, n, k, prepared, out_dtype):
+    g = 128
+    print(f"w4a8 grouped few rows m={m} n={n} k={k} prepared={prepared} out={out_dtype}", flush=True)
+    x = activations(m, k, 1300 + m)
+    qd, gs, bias = packed_int4(n, k, 1301 + n), group_scales(k, n, g, 1302), bf16_vec(n, 1303, 0.01)
+    qdd = qd.to(dev)
+    y = _mx().w4a8_grouped_linear(x.to(dev), _mx().prepare_w4a8_grouped(qdd) if prepared else qdd, gs.to(dev), g,
+                                  bias=bias.to(dev), out_dtype=out_dtype)
+    a, xs = eager_np.quantize_int8_rowwise(bits(x))
+    code = {torch.bfloat16: "bf16", torch.float16: "fp16", torch.float32: "fp32"}[out_dtype]
+    ref = eager_np.w4a8_grouped_linear(a, xs, qd.numpy(), gs.numpy(), g, bits(bias), code)
+    assert np.array_equal(y.float().cpu().numpy().view(np.uint32), ref.astype(np.float32).view(np.uint32))

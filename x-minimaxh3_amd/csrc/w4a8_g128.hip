@@ -344,11 +344,189 @@ int launch_tiles(W4Args p, int out_dtype, bool prepared, hipStream_t st) {
   return mxq_check_launch("w4a8_g128_kernel");
 }
 
+// ---- few rows ----
+// A problem of few tiles leaves most CUs idle while each workgroup walks all of K alone, a group per stage (20480 x
+// 5120: 40 workgroups of 160 stages of 0.45 us), and the fp32 fold over the groups, whose order is part of
+// the result, forbids cutting K. Here a workgroup holds 32 columns and 32 kBI rows, and its eight waves
+// multiply eight groups at once, each its own from global memory (every operand byte has one reader; the activations
+// pass through the wave's own LDS, which takes a quarter of the lines per load instruction). The int32
+// group sums meet in LDS, where each wave folds two of the sixteen accumulator registers' outputs over the eight
+// groups in order. Bound by the latency and the lines of its loads (2 TB/s of weights). Prepared weights from HBM, us
+// before and after: 1 x 20480 x 5120 (K x N) 74.5 -> 25.5, 32 x 20480 x 5120 74.6 -> 31.4, 64 x 14336 x 5376 53.0 ->
+// 32.5, 32 x 7168 x 5376 27.8 -> 12.1, 20 x 3072 x 3072 14.2 -> 9.2, 77 x 20480 x 5120 72.9 -> 54.7.
+constexpr int kFewWaves = 8;
+
+// Orders a wave's LDS accesses before the call against those after it (one wave's execute in order).
+MXQ_DEVICE void few_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int kOut, bool kPrepared, int kBI>
+__global__ __launch_bounds__(kFewWaves * 64, 2) void w4a8_g128_few_kernel(W4Args p) {
+  // a wave's activation rows of its group, and then its sums, by the round's parity
+  __shared__ __attribute__((aligned(16))) int32_t s_wave[2][kFewWaves][kBI][16 * 64];
+  __shared__ __attribute__((aligned(16))) float s_scale[2][32][kFewWaves];
+  constexpr int kFewAhead = kBI == 1 ? 4 : 2;  // rounds of eight groups requested ahead (registers bound it)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int lr = lane & 31, lh = lane >> 5;
+  const int64_t m0 = (int64_t)blockIdx.y * 32 * kBI, n0 = (int64_t)blockIdx.x * 32;
+  const int groups = (int)(p.K / 128), rounds = (groups + kFewWaves - 1) / kFewWaves;
+  const int64_t col = n0 + lr, colc = min(col, p.N - 1);
+  // lane half h takes k in [64 h, 64 h + 64) of a group; the launcher guarantees 32-bit offsets
+  // (activations: eight lanes to a row's 128 bytes, which are one line; a lane's fragments are then read from LDS)
+  uint32_t a_off[kBI][4];
+#pragma unroll
+  for (int i = 0; i < kBI; ++i)
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      a_off[i][t] = (uint32_t)(min(m0 + i * 32 + t * 8 + (lane >> 3), p.M - 1) * p.K + (lane & 7) * 16);
+  const uint32_t b_off = (uint32_t)(colc * (p.K / 2) + lh * 32);
+
+  struct Operands {
+    v4i a[kBI][4], b[2];
+    uint16_t scale;
+  };
+  auto load = [&](int round, Operands& o) {  // past the end: the last group again, folded with a scale of 0
+    const int g = min(round * kFewWaves + wave, groups - 1);
+    const int8_t* a = p.a + (int64_t)g * 128;
+    const uint8_t* b = p.w + (int64_t)g * 64;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) o.b[t] = *reinterpret_cast<const v4i*>(b + b_off + t * 16);
+    o.scale = p.gs[(int64_t)g * p.N + colc];
+#pragma unroll
+    for (int i = 0; i < kBI; ++i)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) o.a[i][t] = *reinterpret_cast<const v4i*>(a + a_off[i][t]);
+  };
+
+  float facc[kBI][2] = {};
+  auto step = [&](int round, const Operands& o) {
+    const int buf = round & 1;
+    // chunk c (16 bytes) of row r at chunk c ^ ((r >> 1) & 7) of the row: no bank conflicts either way
+    char* rows = reinterpret_cast<char*>(&s_wave[buf][wave][0][0]);
+#pragma unroll
+    for (int i = 0; i < kBI; ++i)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int r = t * 8 + (lane >> 3);
+        *reinterpret_cast<v4i*>(rows + i * 4096 + r * 128 + (((lane & 7) ^ ((r >> 1) & 7)) << 4)) = o.a[i][t];
+      }
+    few_lds_order();
+    v4i fa[kBI][4];
+#pragma unroll
+    for (int i = 0; i < kBI; ++i)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        fa[i][t] = *reinterpret_cast<const v4i*>(rows + i * 4096 + lr * 128 + (((lh * 4 + t) ^ ((lr >> 1) & 7)) << 4));
+    v16i acc[kBI];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      uint32_t u[4];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const uint32_t w = (uint32_t)o.b[s >> 1][(s & 1) * 2 + h];
+        if constexpr (kPrepared)
+          unpack8_prepared(w, u[2 * h], u[2 * h + 1]);
+        else
+          unpack8(w, u[2 * h], u[2 * h + 1]);
+      }
+      const v4i fb = v4i{(int)u[0], (int)u[1], (int)u[2], (int)u[3]};
+#pragma unroll
+      for (int i = 0; i < kBI; ++i)
+        acc[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i][s], fb, s == 0 ? v16i{} : acc[i], 0, 0, 0);
+    }
+    few_lds_order();  // the rows have been read
+#pragma unroll
+    for (int i = 0; i < kBI; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s_wave[buf][wave][i][r * 64 + lane] = acc[i][r];
+    // (a group past the end changes nothing: fma(sum, 0, f) == f)
+    if (lane < 32) s_scale[buf][lane][wave] = round * kFewWaves + wave < groups ? f16_to_f32(o.scale) : 0.0f;
+    // One barrier a round: round + 2 writes this buffer again, behind the barrier of round + 1, which every
+    // wave reaches only after its fold of this round.
+    wait_lgkm<0>();
+    barrier_no_drain();
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    const v4f sc[2] = {*reinterpret_cast<const v4f*>(&s_scale[buf][lr][0]), *reinterpret_cast<const v4f*>(&s_scale[buf][lr][4])};
+    int32_t sum[kFewWaves][kBI][2];
+#pragma unroll
+    for (int g = 0; g < kFewWaves; ++g)
+#pragma unroll
+      for (int i = 0; i < kBI; ++i)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) sum[g][i][e] = s_wave[buf][g][i][(e * 8 + wave) * 64 + lane];
+#pragma unroll
+    for (int g = 0; g < kFewWaves; ++g)
+#pragma unroll
+      for (int i = 0; i < kBI; ++i)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) facc[i][e] = fmaf((float)sum[g][i][e], sc[g >> 2][g & 3], facc[i][e]);
+  };
+  Operands o[kFewAhead + 1];
+#pragma unroll
+  for (int t = 0; t < kFewAhead; ++t) load(t, o[t]);
+  for (int round = 0; round < rounds; round += kFewAhead + 1) {
+#pragma unroll
+    for (int t = 0; t <= kFewAhead; ++t) {
+      if (round + t < rounds) {  // uniform
+        load(round + t + kFewAhead, o[(t + kFewAhead) % (kFewAhead + 1)]);
+        step(round + t, o[t]);
+      }
+    }
+  }
+
+  typedef typename OutT<kOut>::T OT;
+  const OT* bias = reinterpret_cast<const OT*>(p.bias);
+  const float bv = bias ? OutT<kOut>::load(bias + colc) : -0.0f;
+#pragma unroll
+  for (int i = 0; i < kBI; ++i)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int r = e * 8 + wave;
+      const int64_t row = m0 + i * 32 + (r >> 2) * 8 + lh * 4 + (r & 3);
+      if (row >= p.M || col >= p.N) continue;
+      const float yb = OutT<kOut>::round(facc[i][e] * (p.xs[row] * 0.0625f)) + bv;
+      char* dst = reinterpret_cast<char*>(p.d) + (row * p.ldd + col) * sizeof(OT);
+      if constexpr (sizeof(OT) == 4)
+        *reinterpret_cast<float*>(dst) = yb;
+      else
+        *reinterpret_cast<uint16_t*>(dst) = (uint16_t)(kOut == 1 ? f32_to_f16_bits(yb) : f32_to_bf16_bits(yb));
+    }
+}
+
+template <int kBI>
+int launch_few(const W4Args& p, int out_dtype, bool prepared, hipStream_t st) {
+  const dim3 grid((unsigned)((p.N + 31) / 32), (unsigned)((p.M + 32 * kBI - 1) / (32 * kBI)));
+  constexpr int kThr = kFewWaves * 64;
+  switch (out_dtype * 2 + (prepared ? 1 : 0)) {
+    case MXQ_DTYPE_F32 * 2: w4a8_g128_few_kernel<0, false, kBI><<<grid, kThr, 0, st>>>(p); break;
+    case MXQ_DTYPE_F32 * 2 + 1: w4a8_g128_few_kernel<0, true, kBI><<<grid, kThr, 0, st>>>(p); break;
+    case MXQ_DTYPE_F16 * 2: w4a8_g128_few_kernel<1, false, kBI><<<grid, kThr, 0, st>>>(p); break;
+    case MXQ_DTYPE_F16 * 2 + 1: w4a8_g128_few_kernel<1, true, kBI><<<grid, kThr, 0, st>>>(p); break;
+    case MXQ_DTYPE_BF16 * 2: w4a8_g128_few_kernel<2, false, kBI><<<grid, kThr, 0, st>>>(p); break;
+    case MXQ_DTYPE_BF16 * 2 + 1: w4a8_g128_few_kernel<2, true, kBI><<<grid, kThr, 0, st>>>(p); break;
+    default: return mxq_set_error(MXQ_ERR_UNSUPPORTED, "output dtype code %d", out_dtype);
+  }
+  return mxq_check_launch("w4a8_g128_few_kernel");
+}
+
 }  // namespace
 
 int launch_w4_g128(W4Args p, int out_dtype, bool prepared, hipStream_t st) {
   if (p.M * p.K >= (int64_t)1 << 31 || p.N * (p.K / 2) >= (int64_t)1 << 31 || p.N * (p.K / 128) * 2 >= (int64_t)1 << 31)
     return MXQ_ERR_UNSUPPORTED;  // the caller falls back to the general kernel
+  // Few rows: the kernel whose waves share K, where it fills the CUs in one round of workgroups (64-row ones take
+  // 0.29 us per group, 32-row ones 0.19, against 0.45 of a 64 x 128 tile's), or two rounds of 32-row ones for 65 to
+  // 96 rows. Past that the tiles win (128 x 20480 x 5120 73 against 80 us; 32 rows of 15360 columns 21.8 against 22.3).
+  // Below eight groups a wave would have nothing to do.
+  const int64_t cols32 = (p.N + 31) / 32, few1 = (p.M + 31) / 32 * cols32, few2 = (p.M + 63) / 64 * cols32;
+  if (p.K >= kFewWaves * 128) {
+    if (few1 <= 256) return launch_few<1>(p, out_dtype, prepared, st);
+    if (few2 <= 256) return launch_few<2>(p, out_dtype, prepared, st);
+    if (p.M > 64 && p.M <= 96 && few1 <= 512) return launch_few<1>(p, out_dtype, prepared, st);
+  }
   // 128-row tiles unless they would leave CUs with fewer than two workgroups (256 CUs).
   const int64_t tiles128 = ((p.M + 127) / 128) * ((p.N + kBN - 1) / kBN);
   return tiles128 >= 2 * 256 ? launch_tiles<128>(p, out_dtype, prepared, st)
