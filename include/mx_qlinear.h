@@ -167,7 +167,7 @@ int mxq_int8_gemm_plan(int64_t M, int64_t N, int64_t K, int table_epilogue, int6
 
 /*
  * The tile-rows an M x N x K problem runs instead of that plan's, when it fills the CUs better (GEMMs of up to
- * sixteen rounds of tiles and K >= 2048; the outputs are the same, bit for bit): plan[0] 0 if none, else the rows of
+ * six rounds of tiles and K >= 2048; the outputs are the same, bit for bit): plan[0] 0 if none, else the rows of
  * its short tiles (192 or 128; 256: no short ones), plan[1] tile-rows of 256, plan[2] short tile-rows behind them,
  * plan[3] 1 when the tiles are claimed from the workspace's counters. All tiles have 256 columns. plan holds
  * 4 entries. A problem whose K is cut (mxq_int8_gemm_workspace) runs neither. Host only; no reference counterpart.

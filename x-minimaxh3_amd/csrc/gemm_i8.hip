@@ -1528,8 +1528,9 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int table, int64_t workspace_byt
 // 28672 and M = 140 to 9000, it picks within 0.4 % of the fastest on average and is 7 % faster than 256- and
 // 128-tiles alone. us before and after: 4331 x 5120 x 5120 134 -> 118, 2587 x 5376 x 14336 219 -> 179 (256-row tiles in
 // place of 128 x 128 ones), 3155 x 21504 x 5376 407 -> 331, 7512 x 5120 x 20480 791 -> 662, 333 x 28672 x 5376
-// SwiGLU 80 -> 72. K below 2048 and more than 16 rounds keep the plan above (an empty part of one round in
-// sixteen is 3 % at most); so do deep-ring problems, whose tiles all run at once.
+// SwiGLU 80 -> 72. K below 2048 and more than 6 rounds keep the plan above (the XCDs' different speeds spread the
+// rounds' ends, so that the time follows the tiles rather than the rounds: 7137 x 21504 x 5376, 9.2 rounds, 700 us whole
+// and 706 short); so do deep-ring problems, whose tiles all run at once.
 struct ShortPlan {
   int rows;        // rows of a short tile: 192 or 128; 256: whole 256-tiles in place of 128-tiles; 0: plan_gemm's
   int tiles_m;     // 256-row tile-rows
@@ -1557,7 +1558,7 @@ static int64_t tile_span(int64_t big, int64_t shorts, int c, int64_t cus) {
 static ShortPlan short_plan(int64_t M, int64_t N, int64_t K, int table, const GemmPlan& g, int64_t workspace_bytes) {
   ShortPlan best{};
   const int64_t cus = std::max(1, mxq_cu_count()), tm = (M + 255) / 256, tn = (N + 255) / 256;
-  if (table == kTableGelu || g.deep || K < 2048 || tm > 16 * cus || tm * tn > 16 * cus) return best;
+  if (table == kTableGelu || g.deep || K < 2048 || tm > 6 * cus || tm * tn > 6 * cus) return best;
   const bool counters = workspace_bytes >= kShortQueueBytes;
   const int64_t whole = tile_span(tm * tn, 0, 100, cus);
   int64_t least = whole;
@@ -1569,6 +1570,8 @@ static ShortPlan short_plan(int64_t M, int64_t N, int64_t K, int table, const Ge
       best = ShortPlan{256, (int)tm, 0, counters && tm * tn > cus};
     }
   }
+  // (three in a hundred of the whole tiles' time to spend on the change of height: smaller gains were not seen)
+  const int64_t margin = std::max<int64_t>(2, least * 3 / 100);
   // (the last two rounds' tile-rows: shorter tiles further up gain nothing)
   for (int h = 192; h >= 128; h -= 64)
     for (int64_t r = tm - 1; r >= std::max<int64_t>(0, tm - 2 - 2 * cus / tn); --r) {
@@ -1576,8 +1579,8 @@ static ShortPlan short_plan(int64_t M, int64_t N, int64_t K, int table, const Ge
       const bool queued = r > 0 || rows * tn > cus;
       if (queued && !counters) continue;
       const int64_t t = tile_span(r * tn, rows * tn, h == 192 ? 90 : 68, cus);
-      if (t + 2 < least) {  // (2: the change of tile height, so that ties keep whole tiles)
-        least = t + 2;
+      if (t < least - (best.rows == 192 || best.rows == 128 ? 0 : margin)) {
+        least = t;
         best = ShortPlan{h, (int)r, (int)rows, queued};
       }
     }
