@@ -374,8 +374,9 @@ int mxq_dequant_int4_grouped_to_int8(const int8_t* qdata, const void* s_rel, int
  * ws = s_channel. Few rows (up to 128, or some hundreds; K a multiple of 256, G = 16, 32 or 64, 16-byte
  * aligned tensors) run a GEMM that decodes the weights in registers instead, its int32 partial
  * sums in `workspace`; the outputs are the same. Arguments as mxq_dequant_int4_grouped_to_int8 and mxq_int8_gemm_dequant;
- * out [M, N] of out_dtype, bias [N] of out_dtype or NULL; gemm_workspace / gemm_workspace_bytes
- * are the chunk GEMMs' tile-queue workspace, as for the INT8 GEMMs (NULL, 0: static order).
+ * K at most 131056 (int32 sums); xq and workspace 16-byte aligned; out [M, N] of out_dtype, bias [N] of
+ * out_dtype or NULL; gemm_workspace / gemm_workspace_bytes are the chunk GEMMs' tile-queue workspace, as
+ * for the INT8 GEMMs (NULL, 0: static order). A refused call launches nothing.
  * Replaces: launch_w4a8_codebook_gemm_chunked, CK/backends/cuda/ops/w4a8_gemm.cu:133-164.
  */
 int mxq_w4a8_codebook_gemm(const int8_t* xq, const int8_t* qdata, const void* s_rel,

@@ -363,3 +363,33 @@ def test_short_tile_plan_covers_every_row(lib, n, table):
             assert p["queued"] or p["rows"] == 256 or (p["tiles_m"] == 0 and p["short_m"] * -(-n // 256) <= 256)
     assert n < 3072 or len(seen) > 1
     assert _lib.gemm_short_plan(4097, 21504, 2032)["rows"] == 0  # short K keeps the uniform tiles
+
+
+@pytest.mark.parametrize("entry", ["mxq_w4a8_codebook_gemm", "mxq_w4a8_codebook_gemm_noalloc"])
+@pytest.mark.parametrize("change,code", [
+    (dict(xq=0), "INVALID"),                     # no activation
+    (dict(xq=264), "UNSUPPORTED"),               # activation not 16-byte aligned
+    (dict(k=131072, chunk=16), "UNSUPPORTED"),   # K beyond the int32 accumulator bound, a multiple of 256
+    (dict(k=1 << 20, chunk=16), "UNSUPPORTED"),
+    (dict(out_dtype=7), "UNSUPPORTED"),
+    (dict(work=264), "UNSUPPORTED"),             # decode workspace not 16-byte aligned
+    (dict(gemm_work=4096 + 64, gemm_bytes=4096), "INVALID"),
+    (dict(gemm_work=4096, gemm_bytes=-1), "INVALID"),
+])
+@pytest.mark.parametrize("m,g", [(1, 16), (128, 64), (1000, 16)])  # few rows (decoded in registers) and many
+def test_codebook_gemm_rejects_before_any_launch(lib, entry, change, code, m, g):
+    """What the decode + GEMM route refuses is refused on every route, with nothing launched."""
+    from mx_qlinear import _lib
+
+    a = dict(xq=256, k=512, chunk=300, out_dtype=_lib.DTYPE_BF16, work=256, gemm_work=0, gemm_bytes=0)
+    a.update(change)
+    if entry.endswith("noalloc") and set(change) & {"work", "gemm_work"}:
+        pytest.skip("the entry has no workspace arguments")
+    d = 256  # never dereferenced: every case is rejected on the host
+    head = (a["xq"] or None, d, d, _lib.DTYPE_F32, None, d, d, None)
+    tail = (d, m, 300, a["k"], g, a["chunk"], a["out_dtype"])
+    if entry.endswith("noalloc"):
+        rc = getattr(lib, entry)(*head, *tail, None)
+    else:
+        rc = getattr(lib, entry)(*head, a["work"], *tail, a["gemm_work"] or None, a["gemm_bytes"], None)
+    assert rc == getattr(_lib, "MXQ_ERR_" + code), lib.mxq_last_error()

@@ -1832,7 +1832,7 @@ static int launch_gemm(const GemmArgs& args0, void* workspace, int64_t workspace
 }
 
 // The tile-queue workspace: NULL (static order) or 256-byte aligned.
-static int check_workspace(const void* workspace, int64_t workspace_bytes) {
+int check_gemm_workspace(const void* workspace, int64_t workspace_bytes) {
   if (!workspace) return MXQ_OK;
   if (workspace_bytes < 0) return mxq_set_error(MXQ_ERR_INVALID, "negative workspace size");
   if ((uintptr_t)workspace % 256) return mxq_set_error(MXQ_ERR_INVALID, "GEMM workspace must be 256-byte aligned");
@@ -1846,7 +1846,7 @@ static int check_gemm_shape(const int8_t* a, const int8_t* b, const void* d, int
   if (ldd < N) return mxq_set_error(MXQ_ERR_INVALID, "output stride %lld < N %lld", (long long)ldd, (long long)N);
   if (M > 0 && N > 0 && K == 0) return mxq_set_error(MXQ_ERR_UNSUPPORTED, "K == 0");
   if (K % 16 != 0) return mxq_set_error(MXQ_ERR_UNSUPPORTED, "K=%lld must be a multiple of 16", (long long)K);
-  if (K > 131056) return mxq_set_error(MXQ_ERR_UNSUPPORTED, "K=%lld exceeds the int32 accumulator bound", (long long)K);
+  if (K > kGemmMaxK) return mxq_set_error(MXQ_ERR_UNSUPPORTED, "K=%lld exceeds the int32 accumulator bound", (long long)K);
   if ((uintptr_t)a % 16 || (uintptr_t)b % 16) return mxq_set_error(MXQ_ERR_UNSUPPORTED, "A and B must be 16-byte aligned");
   return MXQ_OK;
 }
@@ -1904,7 +1904,7 @@ extern "C" int mxq_int8_gemm_i32(const int8_t* a, const int8_t* b, int32_t* c, i
                                  int64_t N, int64_t K, int64_t ldc, void* workspace,
                                  int64_t workspace_bytes, void* stream) {
   int rc = check_gemm_shape(a, b, c, M, N, K, ldc);
-  if (!rc) rc = check_workspace(workspace, workspace_bytes);
+  if (!rc) rc = check_gemm_workspace(workspace, workspace_bytes);
   if (rc) return rc;
   if (M == 0 || N == 0) return MXQ_OK;
   GemmArgs g{};
@@ -1917,7 +1917,7 @@ extern "C" int mxq_int8_gemm_dequant(const int8_t* a, const int8_t* b, const flo
                                      int64_t M, int64_t N, int64_t K, int64_t ldd, int out_dtype,
                                      void* workspace, int64_t workspace_bytes, void* stream) {
   int rc = check_gemm_shape(a, b, d, M, N, K, ldd);
-  if (!rc) rc = check_workspace(workspace, workspace_bytes);
+  if (!rc) rc = check_gemm_workspace(workspace, workspace_bytes);
   if (rc) return rc;
   if (M == 0 || N == 0) return MXQ_OK;
   if (!xs || !ws) return mxq_set_error(MXQ_ERR_INVALID, "null scale pointer");
@@ -1942,7 +1942,7 @@ extern "C" int mxq_int8_gemm_dequant_gelu_absmax(const int8_t* a, const int8_t* 
                                                  int64_t K, int64_t ldh, void* workspace,
                                                  int64_t workspace_bytes, void* stream) {
   int rc = check_gemm_shape(a, b, h_bf16, M, N, K, ldh);
-  if (!rc) rc = check_workspace(workspace, workspace_bytes);
+  if (!rc) rc = check_gemm_workspace(workspace, workspace_bytes);
   if (rc) return rc;
   if (M == 0 || N == 0) return MXQ_OK;
   if (!xs || !ws || !row_absmax) return mxq_set_error(MXQ_ERR_INVALID, "null pointer");
@@ -1959,7 +1959,7 @@ extern "C" int mxq_int8_gemm_dequant_swiglu(const int8_t* a, const int8_t* b, co
                                             void* workspace, int64_t workspace_bytes, void* stream) {
   if (N % 32) return mxq_set_error(MXQ_ERR_INVALID, "SwiGLU fc1 width %lld must be a multiple of 32", (long long)N);
   int rc = check_gemm_shape(a, b, h_bf16, M, N / 2, K, ldh);
-  if (!rc) rc = check_workspace(workspace, workspace_bytes);
+  if (!rc) rc = check_gemm_workspace(workspace, workspace_bytes);
   if (rc) return rc;
   if (M == 0 || N == 0) return MXQ_OK;
   if (!xs || !ws) return mxq_set_error(MXQ_ERR_INVALID, "null pointer");
@@ -1977,7 +1977,7 @@ extern "C" int mxq_int8_gemm_gated_residual(const int8_t* a, const int8_t* b, co
                                             int64_t M, int64_t N, int64_t K, void* workspace,
                                             int64_t workspace_bytes, void* stream) {
   int rc = check_gemm_shape(a, b, residual_bf16, M, N, K, ldr);
-  if (!rc) rc = check_workspace(workspace, workspace_bytes);
+  if (!rc) rc = check_gemm_workspace(workspace, workspace_bytes);
   if (rc) return rc;
   if (M == 0 || N == 0) return MXQ_OK;
   if (!xs || !ws || !gate_bf16 || !gate_rows) return mxq_set_error(MXQ_ERR_INVALID, "null pointer");

@@ -371,7 +371,7 @@ static int codebook_gemm_chunks(const int8_t* xq, const int8_t* qdata, const voi
   hipStream_t st = (hipStream_t)stream;
   const W4RefArgs ref{xq, (const uint8_t*)qdata, s_rel, codebook, M, N, K, s_rel_dtype == MXQ_DTYPE_E4M3, (int)group_size};
   const W4RefPlan plan = plan_w4_ref(ref, std::min(chunk_cols, N) * K);
-  if (plan.rows && (uintptr_t)workspace % 16 == 0) {
+  if (plan.rows) {
     const int rc = launch_w4_ref(ref, plan, reinterpret_cast<int32_t*>(workspace), st);
     if (rc) return rc;
     return launch_split_dequant(reinterpret_cast<const int32_t*>(workspace), plan.splits, plan.ldp, xs, s_channel, bias, out,
@@ -390,15 +390,21 @@ static int codebook_gemm_chunks(const int8_t* xq, const int8_t* qdata, const voi
   return MXQ_OK;
 }
 
-static int check_codebook_gemm(const int8_t* qdata, const void* s_rel, int s_rel_dtype,
+// Everything that either route would refuse is refused here, before a launch: the few-row GEMM has no checks of its
+// own, and the decode of a chunk runs ahead of the GEMM that has them (limits as in mxq_int8_gemm_dequant).
+static int check_codebook_gemm(const int8_t* xq, const int8_t* qdata, const void* s_rel, int s_rel_dtype,
                                const float* s_channel, const float* xs, const void* out, int64_t M,
-                               int64_t N, int64_t K, int64_t group_size, int64_t chunk_cols) {
+                               int64_t N, int64_t K, int64_t group_size, int64_t chunk_cols, int out_dtype) {
   int rc = check_decode_args(qdata, s_rel, s_rel_dtype, N, K, group_size);
   if (rc) return rc;
   if (M < 0) return mxq_set_error(MXQ_ERR_INVALID, "negative M");
   if (M == 0 || N == 0) return MXQ_OK;
   if (chunk_cols <= 0) return mxq_set_error(MXQ_ERR_INVALID, "chunk_cols must be positive");
-  if (!out || !s_channel || !xs) return mxq_set_error(MXQ_ERR_INVALID, "null pointer");
+  if (!xq || !out || !s_channel || !xs) return mxq_set_error(MXQ_ERR_INVALID, "null pointer");
+  if (K > kGemmMaxK) return mxq_set_error(MXQ_ERR_UNSUPPORTED, "K=%lld exceeds the int32 accumulator bound", (long long)K);
+  if ((uintptr_t)xq % 16) return mxq_set_error(MXQ_ERR_UNSUPPORTED, "the activation must be 16-byte aligned");
+  if (out_dtype != MXQ_DTYPE_F32 && out_dtype != MXQ_DTYPE_F16 && out_dtype != MXQ_DTYPE_BF16)
+    return mxq_set_error(MXQ_ERR_UNSUPPORTED, "output dtype code %d", out_dtype);
   return MXQ_OK;
 }
 
@@ -409,9 +415,13 @@ extern "C" int mxq_w4a8_codebook_gemm(const int8_t* xq, const int8_t* qdata, con
                                       int64_t K, int64_t group_size, int64_t chunk_cols,
                                       int out_dtype, void* gemm_workspace, int64_t gemm_workspace_bytes,
                                       void* stream) {
-  int rc = check_codebook_gemm(qdata, s_rel, s_rel_dtype, s_channel, xs, out, M, N, K, group_size, chunk_cols);
+  int rc = check_codebook_gemm(xq, qdata, s_rel, s_rel_dtype, s_channel, xs, out, M, N, K, group_size, chunk_cols,
+                               out_dtype);
   if (rc || M == 0 || N == 0) return rc;
   if (!workspace) return mxq_set_error(MXQ_ERR_INVALID, "null workspace");
+  if ((uintptr_t)workspace % 16) return mxq_set_error(MXQ_ERR_UNSUPPORTED, "the decode workspace must be 16-byte aligned");
+  rc = check_gemm_workspace(gemm_workspace, gemm_workspace_bytes);
+  if (rc) return rc;
   return codebook_gemm_chunks(xq, qdata, s_rel, s_rel_dtype, codebook, s_channel, xs, bias, workspace, out, M, N,
                               K, group_size, chunk_cols, out_dtype, gemm_workspace, gemm_workspace_bytes, stream);
 }
@@ -479,7 +489,8 @@ extern "C" int mxq_w4a8_codebook_gemm_noalloc(const int8_t* xq, const int8_t* qd
                                               const float* s_channel, const float* xs, const void* bias,
                                               void* out, int64_t M, int64_t N, int64_t K, int64_t group_size,
                                               int64_t chunk_cols, int out_dtype, void* stream) {
-  int rc = check_codebook_gemm(qdata, s_rel, s_rel_dtype, s_channel, xs, out, M, N, K, group_size, chunk_cols);
+  int rc = check_codebook_gemm(xq, qdata, s_rel, s_rel_dtype, s_channel, xs, out, M, N, K, group_size, chunk_cols,
+                               out_dtype);
   if (rc || M == 0 || N == 0) return rc;
   const int64_t cols = chunk_cols < N ? chunk_cols : N;
   if (cols > kNoAllocScratchBytes / K)

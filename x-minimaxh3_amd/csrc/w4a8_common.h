@@ -130,6 +130,11 @@ struct W4RefPlan {
 W4RefPlan plan_w4_ref(const W4RefArgs& p, int64_t room);
 int launch_w4_ref(const W4RefArgs& p, const W4RefPlan& plan, int32_t* part, hipStream_t st);
 
+// The INT8 GEMMs' limits (gemm_i8.hip): the largest K whose int32 sums cannot wrap (128 * 128 * K < 2^31), and the
+// check of a tile-queue workspace (NULL or 256-byte aligned, no negative size).
+constexpr int64_t kGemmMaxK = 131056;
+int check_gemm_workspace(const void* workspace, int64_t workspace_bytes);
+
 // Sums `splits` slices of partial results [M, ldp] and applies the dequant epilogue (gemm_i8.hip).
 int launch_split_dequant(const int32_t* part, int splits, int64_t ldp, const float* xs, const float* ws, const void* bias,
                          void* d, int64_t M, int64_t N, int64_t ldd, int out_dtype, hipStream_t st);
