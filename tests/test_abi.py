@@ -371,6 +371,7 @@ def test_short_tile_plan_covers_every_row(lib, n, table):
     (dict(xq=264), "UNSUPPORTED"),               # activation not 16-byte aligned
     (dict(k=131072, chunk=16), "UNSUPPORTED"),   # K beyond the int32 accumulator bound, a multiple of 256
     (dict(k=1 << 20, chunk=16), "UNSUPPORTED"),
+    (dict(k=0), "UNSUPPORTED"),                  # K == 0 with a non-empty output
     (dict(out_dtype=7), "UNSUPPORTED"),
     (dict(work=264), "UNSUPPORTED"),             # decode workspace not 16-byte aligned
     (dict(gemm_work=4096 + 64, gemm_bytes=4096), "INVALID"),

@@ -401,6 +401,7 @@ static int check_codebook_gemm(const int8_t* xq, const int8_t* qdata, const void
   if (M == 0 || N == 0) return MXQ_OK;
   if (chunk_cols <= 0) return mxq_set_error(MXQ_ERR_INVALID, "chunk_cols must be positive");
   if (!xq || !out || !s_channel || !xs) return mxq_set_error(MXQ_ERR_INVALID, "null pointer");
+  if (K == 0) return mxq_set_error(MXQ_ERR_UNSUPPORTED, "K == 0");
   if (K > kGemmMaxK) return mxq_set_error(MXQ_ERR_UNSUPPORTED, "K=%lld exceeds the int32 accumulator bound", (long long)K);
   if ((uintptr_t)xq % 16) return mxq_set_error(MXQ_ERR_UNSUPPORTED, "the activation must be 16-byte aligned");
   if (out_dtype != MXQ_DTYPE_F32 && out_dtype != MXQ_DTYPE_F16 && out_dtype != MXQ_DTYPE_BF16)
