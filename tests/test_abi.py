@@ -394,3 +394,60 @@ def test_codebook_gemm_rejects_before_any_launch(lib, entry, change, code, m, g)
     else:
         rc = getattr(lib, entry)(*head, a["work"], *tail, a["gemm_work"] or None, a["gemm_bytes"], None)
     assert rc == getattr(_lib, "MXQ_ERR_" + code), lib.mxq_last_error()
+
+
+@pytest.mark.parametrize("m", [1, 2, 32, 33, 64, 65, 77, 128, 129, 300, 1000, 4096, 20000])
+def test_split_problems_use_no_counters(lib, m):
+    """A problem whose K the library splits is given memory whose counters are not cleared; neither it, run with
+    less room, nor a narrower problem in the same memory (a last column chunk) has a plan that claims tiles."""
+    from mx_qlinear import _lib
+
+    seen = 0
+    for n in (1, 96, 128, 500, 1024, 3072, 5120, 5376, 14336, 21504, 28672, 32768):
+        for k in (512, 2048, 2064, 5376, 7168, 14336, 20480, 131056):
+            need = _lib.gemm_workspace_bytes(m, n, k)
+            if need <= _lib.GEMM_WORKSPACE_BYTES:
+                continue
+            seen += 1
+            for cols in {1, n // 7 + 1, n // 2 + 1, max(1, n - 129), max(1, n - 1), n}:
+                assert _lib.gemm_plan(m, cols, k, 0, need)["pool"] == 0, (n, k, cols)
+                assert not _lib.gemm_short_plan(m, cols, k, 0, need)["queued"], (n, k, cols)
+    assert seen > 0 or m > 4000
+
+
+def test_gemm_workspace_is_asked_for_on_the_launch_device(monkeypatch):
+    """The plan fills the CUs of the device that the launch runs on: its workspace is asked for with that device
+    current, and one device's answer is not another's (two devices of different plans, stood in for)."""
+    import contextlib
+
+    import torch
+
+    from mx_qlinear import _lib, ops
+
+    current, asked = [0], []
+
+    @contextlib.contextmanager
+    def device(d):
+        before, current[0] = current[0], torch.device(d).index
+        yield
+        current[0] = before
+
+    def query(name, m, n, k, table, out):
+        asked.append(current[0])
+        out._obj.value = 0 if current[0] else _lib.GEMM_WORKSPACE_BYTES
+
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: current[0])
+    monkeypatch.setattr(torch.cuda, "device", device)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(_lib, "call", query)
+    monkeypatch.setattr(ops, "_raw_stream", lambda index: 7)
+    kept = torch.zeros(_lib.GEMM_WORKSPACE_BYTES, dtype=torch.uint8)
+    monkeypatch.setattr(ops, "_GEMM_WORKSPACES", {(0, 7): kept})
+    _lib.gemm_workspace_bytes.cache_clear()
+    try:
+        for _ in range(2):  # asked, then kept
+            assert ops._gemm_ws(torch.device("cuda:0"), 4097, 21504, 5376)[1] == _lib.GEMM_WORKSPACE_BYTES
+            assert ops._gemm_ws(torch.device("cuda:1"), 4097, 21504, 5376) == (None, 0)
+        assert asked == [0, 1] and current[0] == 0
+    finally:
+        _lib.gemm_workspace_bytes.cache_clear()

@@ -124,9 +124,10 @@ def gemm_short_plan(m: int, n: int, k: int, table: int = 0, workspace_bytes: int
 
 
 @functools.lru_cache(maxsize=4096)
-def gemm_workspace_bytes(m: int, n: int, k: int, table: int = 0) -> int:
+def gemm_workspace_bytes(m: int, n: int, k: int, table: int = 0, device: int | None = None) -> int:
     """Workspace an INT8 GEMM of this shape can use (mxq_int8_gemm_workspace): none, the tile-queue
-    counters, or those with room for the partial sums of a K split."""
+    counters, or those with room for the partial sums of a K split. The library answers for the current
+    device, whose CUs its plans fill; ``device`` is that device's index, so that answers are kept apart."""
     out = ctypes.c_int64()
     call("mxq_int8_gemm_workspace", m, n, k, int(table), ctypes.byref(out))
     return out.value

@@ -77,10 +77,15 @@ def _gemm_ws(device: torch.device, m: int = 0, n: int = 0, k: int = 0, table: in
     captured graph shares no memory with eager calls.
 
     A problem of few tiles, whose K the library splits, gets room for its partial sums instead: a
-    tensor of this call's own (it uses no counters), which the returned pointer keeps alive until the
-    launch."""
+    tensor of this call's own, which the returned pointer keeps alive until the launch. Its first
+    GEMM_WORKSPACE_BYTES, where other launches keep their counters, are not cleared: a problem that splits
+    uses none, nor does a narrower one given the same workspace (a last column chunk). That holds for the plan of
+    the device the launch runs on, so the library is asked with that device current."""
+    if torch.cuda.current_device() != device.index:
+        with torch.cuda.device(device):
+            return _gemm_ws(device, m, n, k, table)
     if m:
-        need = _lib.gemm_workspace_bytes(m, n, k, table)
+        need = _lib.gemm_workspace_bytes(m, n, k, table, device.index)
         if need == 0:  # neither a queue nor a split
             return None, 0
         if need > _lib.GEMM_WORKSPACE_BYTES:
@@ -88,9 +93,8 @@ def _gemm_ws(device: torch.device, m: int = 0, n: int = 0, k: int = 0, table: in
             ptr = _p(part)
             ptr.keep = part
             return ptr, need
-    with torch.cuda.device(device):
-        if torch.cuda.is_current_stream_capturing():
-            return None, 0
+    if torch.cuda.is_current_stream_capturing():
+        return None, 0
     key = (device.index, _raw_stream(device.index))
     ws = _GEMM_WORKSPACES.get(key)
     if ws is None:
