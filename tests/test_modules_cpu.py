@@ -56,3 +56,19 @@ def test_int8_weight_stays_the_stored_tensor_when_no_padding_is_needed():
     w = torch.zeros(64, 1024, dtype=torch.int8)
     layer = _layer()
     assert layer.qweight.shape == w.shape and not hasattr(layer.qweight, "_mxq_gemm_weight")
+
+
+def test_package_imports_on_a_cpu_build_of_torch():
+    """Checkpoint and module code runs where torch has no GPU functions at all; they are looked up when called."""
+    import pathlib
+    import subprocess
+    import sys
+
+    code = ("import torch\n"
+            "for name in [n for n in dir(torch._C) if n.startswith('_cuda_')]:\n"
+            "    delattr(torch._C, name)\n"
+            "import mx_qlinear, mx_qlinear.ops, mx_qlinear.checkpoint, mx_qlinear.modules\n"
+            "print('imported')")
+    pkg = pathlib.Path(__file__).resolve().parents[1] / "x-minimaxh3_amd"
+    run = subprocess.run([sys.executable, "-c", code], cwd=pkg, capture_output=True, text=True, timeout=300)
+    assert run.returncode == 0 and "imported" in run.stdout, run.stderr[-2000:]

@@ -35,7 +35,9 @@ def _stream(device: torch.device):
 # only when it is not the current one, and a factor that is already float32 (or the output dtype),
 # contiguous and in place passes through without a chain of no-op conversions. One int8_linear of two
 # launches: 41 -> 20 us of host time (one row 24 -> 16, the row quantizer alone 15 -> 9).
-_raw_stream = torch._C._cuda_getCurrentRawStream
+def _raw_stream(index: int) -> int:
+    # (looked up when called: a CPU build of torch has no such function and still imports this module)
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def _ptr(t: torch.Tensor | None):
