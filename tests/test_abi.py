@@ -451,3 +451,18 @@ def test_gemm_workspace_is_asked_for_on_the_launch_device(monkeypatch):
         assert asked == [0, 1] and current[0] == 0
     finally:
         _lib.gemm_workspace_bytes.cache_clear()
+
+
+@pytest.mark.parametrize("other", [dict(mxq_of_a_later_version=[]), 99])
+def test_library_of_other_sources_is_refused(lib, monkeypatch, other):
+    """A library that lacks an entry point of this package, or has another ABI version, fails to load with a
+    message that names it and the way to build it again."""
+    from mx_qlinear import _lib
+
+    monkeypatch.setattr(_lib, "_lib", None)
+    if isinstance(other, dict):
+        monkeypatch.setattr(_lib, "SIGNATURES", {**_lib.SIGNATURES, **other})
+    else:
+        monkeypatch.setattr(_lib, "ABI_VERSION", other)
+    with pytest.raises(RuntimeError, match="later_version.*build it again" if isinstance(other, dict) else "expected 99.*build"):
+        _lib.load()

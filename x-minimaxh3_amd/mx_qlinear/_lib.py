@@ -80,7 +80,8 @@ class MxqError(RuntimeError):
 
 
 def load() -> ctypes.CDLL:
-    """Load libmx_qlinear.so once; raise RuntimeError if it has not been built."""
+    """Load libmx_qlinear.so once; raise RuntimeError if it has not been built, or was built from other sources
+    than this package (another ABI version, or an entry point that it lacks)."""
     global _lib
     if _lib is not None:
         return _lib
@@ -96,6 +97,14 @@ def load() -> ctypes.CDLL:
             lib.mxq_last_error.argtypes = []
             lib.mxq_abi_version.restype = ctypes.c_int
             lib.mxq_abi_version.argtypes = []
+            have = lib.mxq_abi_version()
+            missing = [name for name in SIGNATURES if not hasattr(lib, name)]
+            if have != ABI_VERSION or missing:
+                raise RuntimeError(
+                    f"{LIB_PATH} does not match this package (ABI version {have}, expected {ABI_VERSION}"
+                    + (f"; missing {', '.join(missing)}" if missing else "")
+                    + "): build it again with __graft_entry__.build() or `python -m mx_qlinear.build`"
+                )
             for name, args in SIGNATURES.items():
                 fn = getattr(lib, name)
                 fn.restype = ctypes.c_int
