@@ -280,6 +280,9 @@ int mxq_int8_gemv_dequant(const int8_t* xq, const float* xs, const int8_t* w, co
  */
 int mxq_gelu_tanh_bf16(const void* x, void* y, int64_t n, void* stream);
 
+/* Rows up to which mxq_rms_adaln_quantize_int8 leaves its workspace unused (the table's launch costs more than it saves). */
+#define MXQ_RMS_ADALN_TABLE_ROWS 12288
+
 /*
  * RMS adaLN (RMSNorm with weight, then segmented modulation), optionally fused with the ConvRot
  * rotation and the per-row INT8 quantizer:
@@ -290,11 +293,12 @@ int mxq_gelu_tanh_bf16(const void* x, void* y, int64_t n, void* stream);
  *   x bf16 [rows, cols]; norm_weight bf16 [cols]; scale, shift bf16 [mod_count, ld_mod];
  *   mod_rows int32 [rows] (clamped into [0, mod_count)). y_out (bf16 [rows, cols]) and q/scales
  *   are each optional (NULL), not both. cols % 16 == 0, ld_mod % 8 == 0, 16-byte aligned tensors.
- *   workspace (optional, 16-byte aligned): with q set and at least mod_count * ld_mod * 2 bytes,
+ *   workspace (optional, 16-byte aligned): with q set, at least mod_count * ld_mod * 2 bytes, more than
+ *   MXQ_RMS_ADALN_TABLE_ROWS rows, cols a multiple of 256 up to 16384 and group_size up to 256,
  *   bf16(1 + scale) of every modulation row is formed there once per call (one small kernel on
- *   the stream before the main one) and read by the main kernel in place of scale; otherwise each
- *   element forms it. The outputs are the same either way. Calls that share a workspace on two
- *   streams race.
+ *   the stream before the main one) and read by the main kernel in place of scale; otherwise the workspace
+ *   is left as it is and each element forms the factor. The outputs are the same either way. Calls that
+ *   share a workspace on two streams race.
  * Semantics: rms_adaln, h3serve/native_engine/model/kernels.py:7594-7640 (eager branch) with
  * RMSNorm = F.rms_norm(x, weight.to(x.dtype), eps) (h3serve/native_engine/model/layers.py:33-48).
  * Replaces: segmented_rms_adaln / native_rms_one_pass_adaln

@@ -121,6 +121,7 @@ def test_gemm_workspace_size_matches_the_header():
     assert "#define MXQ_GEMM_WORKSPACE_BYTES ((int64_t)4096)" in text
     assert _lib.GEMM_WORKSPACE_BYTES == 4096
     assert f"#define MXQ_ABI_VERSION {_lib.ABI_VERSION}" in text
+    assert f"#define MXQ_RMS_ADALN_TABLE_ROWS {_lib.RMS_ADALN_TABLE_ROWS}" in text
 
 
 def test_python_maps_codes_to_the_reference_exceptions(lib):

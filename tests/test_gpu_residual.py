@@ -271,3 +271,39 @@ def test_rms_adaln_modulation_workspace_changes_nothing(dev, m, ld_pad):
     # and the modulated rows are the oracle's within the stated bound
     _check_rms_adaln_bound(outs[0][2].cpu(), x.cpu(), w.cpu(), scale[:, :d].contiguous().cpu(), shift[:, :d].contiguous().cpu(),
                            rows.cpu().numpy(), eps)
+
+
+@pytest.mark.parametrize("over", [0, 1])
+def test_rms_adaln_modulation_table_from_many_rows(dev, over):
+    """The workspace holds bf16(1 + scale) after a call of more than RMS_ADALN_TABLE_ROWS rows and is untouched by one
+    of that many; q, scales and y are those of a call without it, for modulation rows strided beyond the hidden size."""
+    from mx_qlinear import _lib
+    from mx_qlinear.ops import _p, _stream
+
+    m, d, eps, mods, ld = _lib.RMS_ADALN_TABLE_ROWS + over, 768, 1e-6, 5, 768 + 40
+    print(f"rms_adaln table m={m} d={d}", flush=True)
+    x, w, _, _ = _rms_inputs(m, d, 95)
+    scale = (0.1 * torch.randn(mods, ld, generator=gen(96))).to(torch.bfloat16).to(dev)
+    shift = (0.1 * torch.randn(mods, ld, generator=gen(97))).to(torch.bfloat16).to(dev)
+    rows = torch.randint(0, mods, (m,), generator=gen(98), dtype=torch.int32).to(dev)
+    x, w = x.to(dev), w.to(dev)
+    outs = []
+    for ws_bytes in (mods * ld * 2, mods * ld * 2 - 16, 0):
+        ws = torch.full((max(ws_bytes, 1),), 0x5A, dtype=torch.uint8, device=dev)
+        q = torch.empty((m, d), dtype=torch.int8, device=dev)
+        s = torch.empty((m, 1), dtype=torch.float32, device=dev)
+        y = torch.empty((m, d), dtype=torch.bfloat16, device=dev)
+        _lib.call("mxq_rms_adaln_quantize_int8", _p(x), _p(w), _p(scale), _p(shift), ld, mods, _p(rows), eps, _p(y),
+                  _p(q), _p(s), m, d, 256, _p(ws) if ws_bytes else None, ws_bytes, _stream(dev))
+        outs.append((q, s, y))
+        if over and ws_bytes == mods * ld * 2:
+            table = ws.view(torch.bfloat16).reshape(mods, ld)[:, :d]
+            assert torch.equal(table, (1 + scale[:, :d].float()).to(torch.bfloat16))
+        else:
+            assert bool((ws == 0x5A).all())
+    for q, s, y in outs[1:]:
+        assert torch.equal(q, outs[0][0]) and torch.equal(s, outs[0][1]) and torch.equal(y, outs[0][2])
+    pick = torch.arange(0, m, 97)
+    qr, sr, _ = cr.convrot_quantize_bf16(bits(outs[0][2][pick.to(dev)].cpu()), 256)
+    assert np.array_equal(outs[0][0][pick.to(dev)].cpu().numpy(), qr)
+    assert np.array_equal(outs[0][1][pick.to(dev)].cpu().numpy().reshape(-1), sr.reshape(-1))

@@ -660,7 +660,7 @@ __global__ __launch_bounds__(256) void swiglu_kernel(const uint16_t* __restrict_
 
 // Rows past which forming the table is worth its launch (5376 columns, two rows of modulation: the table saves 3.0 us
 // of 69.8 at 8000 rows and 6.4 of 131.1 at 16000, its launch takes 4.7).
-constexpr int64_t kTabRows = 12288;
+constexpr int64_t kTabRows = MXQ_RMS_ADALN_TABLE_ROWS;
 
 // t[m, c] = bf16(1 + scale[m, c]) for the modulation rows (c < cols, row stride ld): the factor
 // every token of segment m multiplies its normalized value by, formed once per call instead of

@@ -23,6 +23,8 @@ DTYPE_F32, DTYPE_F16, DTYPE_BF16, DTYPE_E4M3 = 0, 1, 2, 5
 ABI_VERSION = 5
 # MXQ_GEMM_WORKSPACE_BYTES: the INT8 GEMMs' tile-queue workspace (counters)
 GEMM_WORKSPACE_BYTES = 4096
+# MXQ_RMS_ADALN_TABLE_ROWS: rows up to which the RMS adaLN quantizer uses no workspace
+RMS_ADALN_TABLE_ROWS = 12288
 ACT_NONE, ACT_GELU_TANH, ACT_SWIGLU = 0, 1, 2
 
 _P = ctypes.c_void_p

@@ -424,9 +424,12 @@ def _rms_adaln_call(value, norm, shift, scale, segments, quant: bool, group: int
         if x.dtype == torch.float16:
             _launch(dev, "mxq_rms_adaln_quantize_int8_f16", *args)
         else:
-            # room for bf16(1 + scale) of each modulation row, formed once per call
-            ws = torch.empty(sc.shape[0] * sc.stride(0) * 2 if quant else 0, dtype=torch.uint8, device=dev)
-            _launch(dev, "mxq_rms_adaln_quantize_int8", *args, _ptr(ws), ws.numel())
+            # room for bf16(1 + scale) of each modulation row, formed once per call of many rows
+            ws, ws_bytes = None, 0
+            if quant and rows > _lib.RMS_ADALN_TABLE_ROWS:
+                ws_bytes = sc.shape[0] * sc.stride(0) * 2
+                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+            _launch(dev, "mxq_rms_adaln_quantize_int8", *args, _ptr(ws), ws_bytes)
     if not quant:
         return y
     return (q, s, y) if want_y else (q, s)
