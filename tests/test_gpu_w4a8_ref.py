@@ -1,7 +1,7 @@
 """GPU parity of the reference-format int4 routes: the decode through tables of 16 levels against the
 oracle, also for scales and codebooks that are not finite, and the few-row GEMM that decodes in
 registers against the decode + GEMM route (one column per chunk leaves no room for its sums), bit for
-bit."""
+bit, with the workspace read back to see which of the two ran."""
 
 import numpy as np
 import pytest
@@ -45,9 +45,21 @@ def test_decode_levels(dev, n, k, g, codebook, e4m3):
     assert np.array_equal(w8, want)
 
 
-# Both sides of each row block and of the split, ragged columns, one stage, an uneven last slice, several 128-row tiles.
+def _slices(work, acc, n):
+    """How many slices of int32 sums [m, n padded to a multiple of 4] at the front of ``work`` add up to acc; 0: none do."""
+    m, ldp = acc.shape[0], (n + 3) // 4 * 4
+    room = work.numel() // (4 * m * ldp)
+    part = work.reshape(-1)[: 4 * room * m * ldp].view(torch.int32).reshape(room, m, ldp)[:, :, :n].to(torch.int64).cumsum(0)
+    hits = [s + 1 for s in range(room) if torch.equal(part[s], acc)]
+    return hits[0] if hits else 0
+
+
+# Both sides of each row block and of the split, ragged columns, one stage, an uneven last slice, two and three 128-row
+# tiles with one slice and with several. Past 128 rows fp32 scales of group 16 decode to memory by rule; the workspace
+# shows which route ran: the slices' sums, or the decoded weights.
 @pytest.mark.parametrize("m,n,k", [(1, 257, 256), (20, 1000, 2304), (32, 130, 5376), (33, 255, 512), (64, 513, 2816),
-                                   (65, 3, 1024), (128, 300, 4352), (129, 260, 1280), (384, 514, 768)])
+                                   (65, 3, 1024), (128, 300, 4352), (129, 260, 1280), (300, 258, 1536), (384, 514, 1792),
+                                   (384, 130, 5376), (385, 130, 5376)])
 @pytest.mark.parametrize("g,e4m3", [(16, True), (32, True), (64, True), (16, False), (32, False), (64, False)])
 def test_few_row_gemm(dev, m, n, k, g, e4m3):
     print(f"few rows m={m} n={n} k={k} g={g} e4m3={e4m3}", flush=True)
@@ -59,17 +71,21 @@ def test_few_row_gemm(dev, m, n, k, g, e4m3):
     sch = (torch.rand(n, generator=gen(3)) * 1e-3).to(dev)
     cb = CODEBOOK.to(dev)
     bias = bf16_vec(n, 5, 0.01).to(dev) if n % 2 else None
+    w8 = mx.dequantize_int4_grouped_to_int8(qd, s, cb, g)
+    acc = (xq.cpu().double() @ w8.cpu().double().t()).to(torch.int64)  # exact
     outs = []
     for chunk in (n, 1):
-        work = torch.empty((chunk, k), dtype=torch.int8, device=dev)
+        work = torch.full((chunk, k), 0x5A, dtype=torch.int8, device=dev)
         y = torch.zeros((m, n), dtype=torch.bfloat16, device=dev)
         L.call("mxq_w4a8_codebook_gemm", _p(xq), _p(qd), _p(s), L.DTYPE_E4M3 if e4m3 else L.DTYPE_F32, _p(cb), _p(sch),
                _p(xs), _p(bias), _p(work), _p(y), m, n, k, g, chunk, L.DTYPE_BF16, None, 0, _stream(dev))
         outs.append(y)
+        if chunk == n and (m <= 128 or (m <= 384 and (e4m3 or g > 16))):
+            assert _slices(work.cpu(), acc, n) > 0, "the sums of the few-row GEMM are not in the workspace"
+        else:
+            assert torch.equal(work, w8[n - chunk:]), "the last chunk's decoded weights are not in the workspace"
     assert torch.equal(outs[0], outs[1])
-    w8 = mx.dequantize_int4_grouped_to_int8(qd, s, cb, g)
-    acc = (xq.cpu().double() @ w8.cpu().double().t()).float()  # exact: below 2^24
-    want = (acc * (xs.cpu()[:, None] * sch.cpu()[None, :])).to(torch.bfloat16)
+    want = (acc.float() * (xs.cpu()[:, None] * sch.cpu()[None, :])).to(torch.bfloat16)  # (float32 of the sum, rounded once)
     if n % 2:
         want = (want.float() + bias.cpu().float()).to(torch.bfloat16)
     assert torch.equal(outs[0].cpu(), want)
