@@ -320,10 +320,11 @@ def test_correction_through_the_module(dev):
 
 
 # Few rows of group 128: workgroups of 32 columns whose eight waves take eight groups at once, with 32- or 64-row
-# tiles: group counts of one full round, a partial last round and several turns of the operand ring, ragged rows
-# and columns, both layouts, every output type.
+# tiles: group counts of one full round, a partial last round and several turns of the operand ring (49 groups are
+# seven rounds: 64-row tiles in (63, 5384, 6272), 32-row ones in (31, 72, 6272)), ragged rows and columns, both
+# layouts, every output type.
 @pytest.mark.parametrize("m,n,k", [(1, 3000, 1024), (32, 136, 1152), (33, 264, 2176), (64, 4096, 1024), (31, 72, 6272),
-                                   (100, 3072, 1408), (80, 5120, 1152), (257, 136, 5248)])
+                                   (100, 3072, 1408), (80, 5120, 1152), (257, 136, 5248), (63, 5384, 6272)])
 @pytest.mark.parametrize("prepared,out_dtype", [(True, torch.bfloat16), (False, torch.float16), (True, torch.float32)])
 def test_grouped_few_rows(dev, m, n, k, prepared, out_dtype):
     g = 128
