@@ -515,15 +515,20 @@ MXQ_DEVICE void stage_block32(char* buf, const uint32_t* w) {
 // col0 .. col0 + 63): res = bf16(res + y * gate[grow]) with 16-byte accesses; grow[t] is the
 // gate row of row row0 + 8 t + lane / 8. The residual and gate reads are issued before the
 // staging so that their latency overlaps it.
-MXQ_DEVICE void gated_lines(const GemmArgs& p, char* buf, int64_t row0, int64_t col0, const int64_t (&grow)[4],
+MXQ_DEVICE void gated_lines(const GemmArgs& p, char* buf, int64_t row0, int64_t col0, const int32_t (&grow)[4],
                             const uint32_t (&w)[2][8]) {
   const int lane = tid_x() & 63;
   uint16_t* res = p.res + (row0 + (lane >> 3)) * p.ldr + col0 + (lane & 7) * 8;
   v4u r[4], g[4];
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
+    // (the gate's address is formed here: ahead of the epilogue, where the compiler would form all of them, they
+    // would take 32 registers of the 256 through it: 137 spills in the 256-row ping-pong tiles against 10, and
+    // 75600 x 5376 x 14336 5.24 against 4.95 ms, 30000 x 5120 x 5120 0.95 against 0.82)
+    int32_t gr = grow[t];
+    __asm__ volatile("" : "+v"(gr));
     r[t] = *reinterpret_cast<const v4u*>(res + t * 8 * p.ldr);
-    g[t] = *reinterpret_cast<const v4u*>(p.gate + grow[t] * p.ldg + col0 + (lane & 7) * 8);
+    g[t] = *reinterpret_cast<const v4u*>(p.gate + gr * p.ldg + col0 + (lane & 7) * 8);
   }
   stage_blocks16(buf, w);
   wave_lds_sync();
@@ -852,12 +857,12 @@ MXQ_DEVICE void gemm_epilogue(const GemmArgs& p, char* lds, v16i (&acc)[C::kBI][
                 "staging buffers overlap the table, the factors or the end of LDS");
   char* sbuf = lds + kSB + wave * kStageBytes;
   const int64_t pitch = p.ldd * kElem;
-  int64_t grow[kBI] = {};     // kEpiGatedRes: the gate row of each of this lane's rows
-  int64_t grow_rm[kBI][4] = {};  // ... and of the rows it updates in the whole-line form
+  int32_t grow[kBI] = {};     // kEpiGatedRes: the gate row of each of this lane's rows
+  int32_t grow_rm[kBI][4] = {};  // ... and of the rows it updates in the whole-line form
   if constexpr (kEpi == kEpiGatedRes) {
-    auto gate_row = [&](int64_t m) {  // clamped into the gate so a bad row index cannot fault
+    auto gate_row = [&](int64_t m) -> int32_t {  // clamped into the gate so a bad row index cannot fault
       const int64_t gr = p.gate_rows[min(m, p.M - 1)];
-      return gr < 0 ? (int64_t)0 : (gr >= p.gate_count ? p.gate_count - 1 : gr);
+      return (int32_t)(gr < 0 ? (int64_t)0 : (gr >= p.gate_count ? p.gate_count - 1 : gr));
     };
 #pragma unroll
     for (int i = 0; i < kBI; ++i) {
