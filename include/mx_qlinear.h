@@ -139,8 +139,8 @@ int mxq_adaln_quantize_int8_f16(const void* x, const void* scale, const void* sh
 #define MXQ_GEMM_WORKSPACE_BYTES ((int64_t)4096)
 
 /*
- * The workspace an M x N x K GEMM can use, in *bytes (table_epilogue as in mxq_int8_gemm_plan): 0 if
- * none, MXQ_GEMM_WORKSPACE_BYTES for the tile queue, or that plus room for the partial sums of a problem
+ * The workspace an M x N x K GEMM can use, in *bytes (table_epilogue as in mxq_int8_gemm_plan, or 3 for the
+ * gated residual): 0 if none, MXQ_GEMM_WORKSPACE_BYTES for the tile queue, or that plus room for the partial sums of a problem
  * of so few tiles that the library would cut its K into slices to fill the CUs. Such a problem given that
  * much runs two launches, the slices and their sum with the epilogue; given less it runs unsplit, with the
  * same outputs. It uses no counters, and the bytes behind the first MXQ_GEMM_WORKSPACE_BYTES need no
@@ -167,7 +167,8 @@ int mxq_int8_gemm_plan(int64_t M, int64_t N, int64_t K, int table_epilogue, int6
 
 /*
  * The tile-rows an M x N x K problem runs instead of that plan's, when it fills the CUs better (GEMMs of up to
- * six rounds of tiles and K >= 2048; the outputs are the same, bit for bit): plan[0] 0 if none, else the rows of
+ * six rounds of tiles and K >= 2048; the outputs are the same, bit for bit; table_epilogue 3 for the gated residual,
+ * whose tiles cost otherwise): plan[0] 0 if none, else the rows of
  * its short tiles (192 or 128; 256: no short ones), plan[1] tile-rows of 256, plan[2] short tile-rows behind them,
  * plan[3] 1 when the tiles are claimed from the workspace's counters. All tiles have 256 columns. plan holds
  * 4 entries. A problem whose K is cut (mxq_int8_gemm_workspace) runs neither. Host only; no reference counterpart.

@@ -467,3 +467,14 @@ def test_library_of_other_sources_is_refused(lib, monkeypatch, other):
         monkeypatch.setattr(_lib, "ABI_VERSION", other)
     with pytest.raises(RuntimeError, match="later_version.*build it again" if isinstance(other, dict) else "expected 99.*build"):
         _lib.load()
+
+
+@pytest.mark.parametrize("m,n,k,table", [(17254, 1536, 2304, 0), (3158, 8192, 2304, 0), (9000, 3072, 2304, 0),
+                                         (20000, 1024, 2048, 0), (10064, 2560, 2304, 0), (18171, 1024, 2048, 0),
+                                         (4331, 3072, 3072, 3), (1100, 15360, 5120, 3), (7647, 2560, 5376, 3)])
+def test_short_and_gated_problems_keep_the_tiles_that_are_faster(lib, m, n, k, table):
+    """Problems of a short K, and gated residuals, whose uniform tiles measured 10 % and more faster than the short or
+    256-row tiles that costs without an epilogue's share chose."""
+    from mx_qlinear import _lib
+
+    assert _lib.gemm_short_plan(m, n, k, table)["rows"] == 0

@@ -15,8 +15,11 @@ pytestmark = pytest.mark.gpu
 # (m, n, k): rows of the short tile, claimed or not. K in whole stages and with a tail, columns whole and
 # ragged (n % 4 != 0 stores element by element), last tiles of one and of almost all their rows.
 SHAPES = [(513, 16001, 2064, 192, False), (576, 16384, 2048, 192, False), (1044, 21504, 2048, 128, True),
-          (1025, 21506, 2160, 128, True), (8129, 5120, 2064, 192, True), (8192, 4990, 2048, 192, True),
-          (2310, 5120, 2064, 256, False), (5000, 3001, 2176, 256, False)]
+          (1025, 21506, 2160, 128, True), (8129, 5120, 4112, 192, True), (8192, 4990, 4096, 192, True),
+          (2310, 5120, 4112, 256, False), (5000, 3001, 2176, 256, False), (8129, 3001, 2064, 256, True)]
+# The same for the gated residual, whose rule has costs of its own.
+GATED = [(2971, 28333, 2064, 128, True), (907, 24818, 2064, 192, True), (793, 28352, 2064, 192, True),
+         (258, 22467, 7184, 192, False), (390, 25509, 14352, 256, False)]
 
 
 def _case(dev, m, n, k, table=0):
@@ -56,6 +59,11 @@ def test_short_tiles(dev, m, n, k, rows, queued):
         L.call("mxq_int8_gemm_dequant", _p(a), _p(w), _p(xs), _p(ws), n, _p(b), _p(y), m, n, k, n, code, _p(space),
                space.numel(), st)
         assert torch.equal(y, _dequant(acc, xs, ws, bias, dtype))
+    _check_gated(dev, a, w, acc, space, xs, ws, bias)
+
+
+def _check_gated(dev, a, w, acc, space, xs, ws, bias):
+    (m, k), n, st = a.shape, w.shape[0], _stream(dev)
     b, gate = bias.bfloat16(), torch.randn(3, n, generator=gen(6)).bfloat16().to(dev)
     grow = torch.randint(0, 3, (m,), generator=gen(7), dtype=torch.int32).to(dev)
     res = torch.randn(m, n, generator=gen(8)).bfloat16().to(dev)
@@ -66,8 +74,18 @@ def test_short_tiles(dev, m, n, k, rows, queued):
     assert torch.equal(res, want) and int(space.count_nonzero()) == 0
 
 
+@pytest.mark.parametrize("m,n,k,rows,queued", GATED)
+def test_short_gated_residual(dev, m, n, k, rows, queued):
+    print(f"short gated residual m={m} n={n} k={k} rows={rows}", flush=True)
+    case = _case(dev, m, n, k)
+    plan = L.gemm_short_plan(m, n, k, L.PLAN_GATED_RESIDUAL)
+    assert (plan["rows"], plan["queued"]) == (rows, queued), plan
+    for _ in range(2):  # the second launch finds the counters as the first left them
+        _check_gated(dev, *case)
+
+
 @pytest.mark.parametrize("m,f,k,rows,queued", [(333, 14336, 2064, 192, False), (129, 14336, 2048, 128, False),
-                                               (1025, 10752, 2064, 128, True), (1194, 10752, 2048, 192, True)])
+                                               (1025, 10752, 2064, 128, True), (1314, 14336, 2064, 192, True)])
 def test_short_swiglu(dev, m, f, k, rows, queued):
     print(f"short swiglu m={m} f={f} k={k} rows={rows}", flush=True)
     import mx_qlinear as mx

@@ -107,6 +107,8 @@ enum { kEpiI32 = 0, kEpiDequant = 1, kEpiGelu = 2, kEpiGatedRes = 3, kEpiSwiGLU 
 // Table epilogues as plan_gemm sees them: GELU keeps the whole 128 KB table in LDS (four-wave
 // 256-tiles), SwiGLU the 8 KB compact SiLU table (ping-pong 256-tiles).
 enum { kTableGelu = 1, kTableSwiGLU = 2 };
+// The plan queries' code of the gated residual epilogue: no table, costs of its own in short_plan.
+enum { kGatedResidual = 3 };
 
 struct GemmArgs {
   const int8_t* a;
@@ -1527,15 +1529,36 @@ static GemmPlan plan_gemm(int64_t M, int64_t N, int table, int64_t workspace_byt
 // A GEMM of a few rounds of tiles loses the part of its last round that is empty: 4097 x 21504 is 1428 tiles of
 // 256 rows, 5.6 rounds on 256 CUs that take the time of six. Its last tile-rows then run as ping-pong tiles of 192 or 128
 // rows, which the workgroups claim once the 256-row tiles are done, and problems of less than a round may run
-// short tiles only. The rule compares the time the tiles take on the CUs, in hundredths of a round of
-// 256-tiles: a 192-row tile 90, a 128-row one 68 (their stages carry the same weight panel for fewer MFMAs); a
-// round of two 128 x 128 tiles per CU 70, of one 45. Fitted to 100 shapes of K = 3072 to 20480, N = 3072 to
-// 28672 and M = 140 to 9000, it picks within 0.4 % of the fastest on average and is 7 % faster than 256- and
-// 128-tiles alone. us before and after: 4331 x 5120 x 5120 134 -> 118, 2587 x 5376 x 14336 219 -> 179 (256-row tiles in
+// short tiles only. The rule compares the time the tiles take on the CUs (TileCost). us before and after:
+// 4331 x 5120 x 5120 134 -> 118, 2587 x 5376 x 14336 219 -> 179 (256-row tiles in
 // place of 128 x 128 ones), 3155 x 21504 x 5376 407 -> 331, 7512 x 5120 x 20480 791 -> 662, 333 x 28672 x 5376
 // SwiGLU 80 -> 72. K below 2048 and more than 6 rounds keep the plan above (the XCDs' different speeds spread the
 // rounds' ends, so that the time follows the tiles rather than the rounds: 7137 x 21504 x 5376, 9.2 rounds, 700 us whole
 // and 706 short); so do deep-ring problems, whose tiles all run at once.
+
+// Time of a tile as K * per_k / 100 + fixed, in units of a 256-tile's time per K: a 192- and a 128-row tile's stages carry
+// the same weight panel as a 256-row one's for fewer MFMAs; fixed is the first loads and the epilogue. A round of two
+// 128 x 128 tiles per CU, and of one.
+struct TileCost {
+  struct Line {
+    int per_k, fixed;
+    int64_t at(int64_t K) const { return K * per_k / 100 + fixed; }
+  } t256, t192, t128, two, one;
+};
+// From K = 4096 on the fixed part is too small to matter. Fitted to 100 shapes of K = 3072 to 20480, N = 3072 to
+// 28672 and M = 140 to 9000, the rule picks within 0.4 % of the fastest on average and is 7 % faster than 256- and
+// 128-tiles alone.
+constexpr TileCost kTileCost = {{100, 0}, {90, 0}, {68, 0}, {70, 0}, {45, 0}};
+// Below, without it, the rule took short tiles where uniform ones were faster (us with the costs above, with
+// these: 17254 x 1536 x 2304 82 and 71, 3158 x 8192 x 2304 81 and 72, 20000 x 1024 x 2048 63 and 57). Fitted to 325
+// shapes of K = 2048 to 3584 timed in every plan: 1.3 % above the fastest on average before, 0.7 % with these.
+constexpr TileCost kTileCostShortK = {{100, 685}, {92, 705}, {62, 955}, {64, 555}, {42, 0}};
+constexpr int64_t kShortK = 4096;
+// Gated residual: the epilogue also reads and writes the residual, and large tiles do that all at once, with no other
+// workgroup's products beside it (4331 x 3072 x 3072 in 256-row tiles, as the costs above have it, 125 us, in 128 x 128
+// ones 90). Fitted to 420 shapes of K = 2048 to 20480: 5.6 % above the fastest on average with the costs above, 4.8 % with
+// these, and 2 % and more slower than the uniform plan in 7 of them, where it was 75.
+constexpr TileCost kTileCostGated = {{100, 1680}, {77, 1390}, {56, 770}, {60, 120}, {37, 380}};
 struct ShortPlan {
   int rows;        // rows of a short tile: 192 or 128; 256: whole 256-tiles in place of 128-tiles; 0: plan_gemm's
   int tiles_m;     // 256-row tile-rows
@@ -1545,11 +1568,11 @@ struct ShortPlan {
 constexpr int kShortQueueBytes = (kShortCounters + 8 * 32) * 4;
 static_assert(MXQ_GEMM_WORKSPACE_BYTES >= kShortQueueBytes, "workspace holds the short tiles' counters");
 
-// The time of `big` 256-tiles and then `shorts` tiles of cost c on `cus` CUs, each CU taking the next tile when
+// The time of `big` tiles of cost c0 and then `shorts` of cost c on `cus` CUs, each CU taking the next tile when
 // it is free.
-static int64_t tile_span(int64_t big, int64_t shorts, int c, int64_t cus) {
-  const int64_t q = big / cus * 100, late = big % cus;  // `late` CUs have one 256-tile more
-  int64_t end = late ? q + 100 : q, ta = q + c, tb = q + 100 + c;
+static int64_t tile_span(int64_t big, int64_t c0, int64_t shorts, int64_t c, int64_t cus) {
+  const int64_t q = big / cus * c0, late = big % cus;  // `late` CUs have one 256-tile more
+  int64_t end = late ? q + c0 : q, ta = q + c, tb = q + c0 + c;
   while (shorts > 0) {
     const bool first = !late || ta <= tb;
     const int64_t t = first ? ta : tb;
@@ -1560,35 +1583,39 @@ static int64_t tile_span(int64_t big, int64_t shorts, int c, int64_t cus) {
   return end;
 }
 
+// table: as in plan_gemm, or kGatedResidual.
 static ShortPlan short_plan(int64_t M, int64_t N, int64_t K, int table, const GemmPlan& g, int64_t workspace_bytes) {
   ShortPlan best{};
   const int64_t cus = std::max(1, mxq_cu_count()), tm = (M + 255) / 256, tn = (N + 255) / 256;
   if (table == kTableGelu || g.deep || K < 2048 || tm > 6 * cus || tm * tn > 6 * cus) return best;
   const bool counters = workspace_bytes >= kShortQueueBytes;
-  const int64_t whole = tile_span(tm * tn, 0, 100, cus);
+  const TileCost& cost = table == kGatedResidual ? kTileCostGated : K < kShortK ? kTileCostShortK : kTileCost;
+  const int64_t c256 = cost.t256.at(K), whole = tile_span(tm * tn, c256, 0, 0, cus);
   int64_t least = whole;
   if (g.tile == 128) {
     const int64_t tiles = (int64_t)g.tiles_m * g.tiles_n, rest = tiles % (2 * cus);
-    least = tiles / (2 * cus) * 70 + (rest > cus ? 70 : rest ? 45 : 0);
+    least = tiles / (2 * cus) * cost.two.at(K) + (rest > cus ? cost.two.at(K) : rest ? cost.one.at(K) : 0);
     if (whole < least) {
       least = whole;
       best = ShortPlan{256, (int)tm, 0, counters && tm * tn > cus};
     }
   }
   // (three in a hundred of the whole tiles' time to spend on the change of height: smaller gains were not seen)
-  const int64_t margin = std::max<int64_t>(2, least * 3 / 100);
+  const int64_t margin = least * 3 / 100;
   // (the last two rounds' tile-rows: shorter tiles further up gain nothing)
-  for (int h = 192; h >= 128; h -= 64)
+  for (int h = 192; h >= 128; h -= 64) {
+    const int64_t c = h == 192 ? cost.t192.at(K) : cost.t128.at(K);
     for (int64_t r = tm - 1; r >= std::max<int64_t>(0, tm - 2 - 2 * cus / tn); --r) {
       const int64_t rows = (M - 256 * r + h - 1) / h;
       const bool queued = r > 0 || rows * tn > cus;
       if (queued && !counters) continue;
-      const int64_t t = tile_span(r * tn, rows * tn, h == 192 ? 90 : 68, cus);
+      const int64_t t = tile_span(r * tn, c256, rows * tn, c, cus);
       if (t < least - (best.rows == 192 || best.rows == 128 ? 0 : margin)) {
         least = t;
         best = ShortPlan{h, (int)r, (int)rows, queued};
       }
     }
+  }
   return best;
 }
 
@@ -1786,7 +1813,8 @@ static int launch_gemm(const GemmArgs& args0, void* workspace, int64_t workspace
       return launch_split<kEpi, kOut>(args, sp, workspace, stream);
   }
   if constexpr (kEpi != kEpiGelu) {
-    const ShortPlan sh = short_plan(args.M, args.N, args.K, kEpi == kEpiSwiGLU ? kTableSwiGLU : 0, g, workspace ? workspace_bytes : 0);
+    constexpr int kCost = kEpi == kEpiSwiGLU ? kTableSwiGLU : kEpi == kEpiGatedRes ? kGatedResidual : 0;
+    const ShortPlan sh = short_plan(args.M, args.N, args.K, kCost, g, workspace ? workspace_bytes : 0);
     if (sh.rows) {
       args.tiles_m = sh.tiles_m;
       args.tiles_n = (int)((args.N + 255) / 256);
@@ -1862,14 +1890,15 @@ using namespace mxq;
 
 extern "C" int mxq_int8_gemm_workspace(int64_t M, int64_t N, int64_t K, int table_epilogue, int64_t* bytes) {
   if (M < 0 || N < 0 || K < 0 || !bytes) return mxq_set_error(MXQ_ERR_INVALID, "bad GEMM workspace request");
-  if (table_epilogue < 0 || table_epilogue > kTableSwiGLU) return mxq_set_error(MXQ_ERR_INVALID, "table_epilogue must be 0, 1 or 2");
+  if (table_epilogue < 0 || table_epilogue > kGatedResidual) return mxq_set_error(MXQ_ERR_INVALID, "table_epilogue must be 0 to 3");
   *bytes = 0;
   if (M == 0 || N == 0 || K == 0) return MXQ_OK;
-  const SplitPlan s = split_plan(M, N, K, table_epilogue);
+  const int table = table_epilogue == kGatedResidual ? 0 : table_epilogue;
+  const SplitPlan s = split_plan(M, N, K, table);
   if (s.splits)
     *bytes = MXQ_GEMM_WORKSPACE_BYTES + s.bytes;
   else {
-    const GemmPlan g = plan_gemm(M, N, table_epilogue, MXQ_GEMM_WORKSPACE_BYTES);
+    const GemmPlan g = plan_gemm(M, N, table, MXQ_GEMM_WORKSPACE_BYTES);
     const ShortPlan sh = short_plan(M, N, K, table_epilogue, g, MXQ_GEMM_WORKSPACE_BYTES);
     if (sh.rows ? sh.queued : g.pool > 0) *bytes = MXQ_GEMM_WORKSPACE_BYTES;
   }
@@ -1879,8 +1908,9 @@ extern "C" int mxq_int8_gemm_workspace(int64_t M, int64_t N, int64_t K, int tabl
 extern "C" int mxq_int8_gemm_short_plan(int64_t M, int64_t N, int64_t K, int table_epilogue,
                                         int64_t workspace_bytes, int64_t* plan) {
   if (M <= 0 || N <= 0 || K <= 0 || !plan) return mxq_set_error(MXQ_ERR_INVALID, "GEMM plan needs a positive shape and an output");
-  if (table_epilogue < 0 || table_epilogue > kTableSwiGLU) return mxq_set_error(MXQ_ERR_INVALID, "table_epilogue must be 0, 1 or 2");
-  const ShortPlan sh = short_plan(M, N, K, table_epilogue, plan_gemm(M, N, table_epilogue, workspace_bytes), workspace_bytes);
+  if (table_epilogue < 0 || table_epilogue > kGatedResidual) return mxq_set_error(MXQ_ERR_INVALID, "table_epilogue must be 0 to 3");
+  const ShortPlan sh = short_plan(M, N, K, table_epilogue, plan_gemm(M, N, table_epilogue == kGatedResidual ? 0 : table_epilogue, workspace_bytes),
+                                  workspace_bytes);
   plan[0] = sh.rows;
   plan[1] = sh.tiles_m;
   plan[2] = sh.short_m;

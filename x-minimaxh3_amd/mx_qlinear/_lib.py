@@ -25,6 +25,7 @@ ABI_VERSION = 5
 GEMM_WORKSPACE_BYTES = 4096
 # MXQ_RMS_ADALN_TABLE_ROWS: rows up to which the RMS adaLN quantizer uses no workspace
 RMS_ADALN_TABLE_ROWS = 12288
+PLAN_GATED_RESIDUAL = 3  # table_epilogue of the gated residual's plan queries
 ACT_NONE, ACT_GELU_TANH, ACT_SWIGLU = 0, 1, 2
 
 _P = ctypes.c_void_p

@@ -848,7 +848,8 @@ def int8_linear_gated_residual_(residual: torch.Tensor, x: torch.Tensor, weight:
         q, xs = quantize_int8_rowwise(x2, input_act=input_act)
     q2, w2, k = _pad_k(q, weight)
     _launch(dev, "mxq_int8_gemm_gated_residual", _ptr(q2), _ptr(w2), _ptr(xs), _ptr(ws), ws.numel(), _ptr(b), _ptr(res2),
-            res2.stride(0), _ptr(g), g.stride(0), g.shape[0], _ptr(gr), rows, n, k, *_gemm_ws(dev, rows, n, k))
+            res2.stride(0), _ptr(g), g.stride(0), g.shape[0], _ptr(gr), rows, n, k,
+            *_gemm_ws(dev, rows, n, k, _lib.PLAN_GATED_RESIDUAL))
     return residual
 
 
