@@ -68,9 +68,8 @@ __global__ __launch_bounds__(256) void decode_int4_grouped_kernel(
       const uint32_t c = (i & 1) ? (byte >> 4) : (byte & 0xFu);
       const int j = i >> gshift;
       const float s = j == 0 ? sv[0] : (j == 1 ? sv[1] : (j == 2 ? sv[2] : sv[3]));
-      float r = __builtin_rintf(s_cb[c] * s);
-      r = fminf(fmaxf(r, -127.0f), 127.0f);
-      const int q = (r != r) ? 0 : (int)r;
+      const float p = s_cb[c] * s;  // (tested ahead of the clamp, which would make a NaN of it -127)
+      const int q = p != p ? 0 : (int)fminf(fmaxf(__builtin_rintf(p), -127.0f), 127.0f);
       o[i >> 2] |= (uint32_t)(q & 0xFF) << (8 * (i & 3));
     }
     *reinterpret_cast<v4u*>(out + n * (k_half * 2) + k0) = v4u{o[0], o[1], o[2], o[3]};
