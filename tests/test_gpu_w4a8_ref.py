@@ -30,7 +30,9 @@ def _scales(n, groups, e4m3, seed):
 
 @pytest.mark.parametrize("e4m3", [False, True])
 @pytest.mark.parametrize("codebook", ["none", "finite", "inf"])
-@pytest.mark.parametrize("n,k,g", [(7, 272, 4), (5, 160, 8), (1, 16, 16), (5, 1040, 16), (3, 4112, 16), (9, 1536, 48), (70, 2048, 64)])
+# Few weights; many by levels in whole rows of one piece and of several, and in pieces of rows (the last of one vector).
+@pytest.mark.parametrize("n,k,g", [(7, 272, 4), (5, 160, 8), (1, 16, 16), (5, 1040, 16), (3, 4112, 16), (9, 1536, 48), (70, 2048, 64),
+                                   (6800, 1552, 16), (4099, 4112, 16), (1281, 8208, 48)])
 def test_decode_levels(dev, n, k, g, codebook, e4m3):
     qd, s = packed_int4(n, k, k + g), _scales(n, k // g, e4m3, n + k)
     cb = None if codebook == "none" else CODEBOOK.clone()

@@ -41,19 +41,25 @@ __global__ __launch_bounds__(256) void decode_int4_grouped_kernel(
     const float* __restrict__ codebook, int8_t* __restrict__ out, int64_t total_vec,
     int64_t k_half, int64_t groups, int group_size, int gshift) {
   __shared__ float s_cb[16];
-  if (threadIdx.x < 16) s_cb[threadIdx.x] = codebook ? codebook[threadIdx.x] : (float)threadIdx.x - 8.0f;
+  __shared__ int s_nan;  // the codebook has an infinity or a NaN
+  if (threadIdx.x < kWave) {
+    const float v = threadIdx.x >= 16 ? 0.0f : codebook ? codebook[threadIdx.x] : (float)threadIdx.x - 8.0f;
+    if (threadIdx.x < 16) s_cb[threadIdx.x] = v;
+    const bool off = __builtin_amdgcn_ballot_w64(!(fabsf(v) < INFINITY)) != 0;
+    if (threadIdx.x == 0) s_nan = off;
+  }
   __syncthreads();
   for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < total_vec;
        v += (int64_t)gridDim.x * blockDim.x) {
     // 8 packed bytes -> 16 weights of one row (K % 16 == 0 keeps them in one row).
-    // The vector's 16 weights lie in 16 / G groups (G = 4, 8): their scales are read once per vector, and
-    // weight i takes scale i >> gshift (gshift = log2 G), so no division runs per weight.
+    // The vector's 16 weights lie in 16 / G groups (G = 4, 8) or in one: their scales are read once per vector, and
+    // weight i takes scale i >> gshift (log2 G, or 4 from G = 16 on), so no division runs per weight.
     const int64_t byte0 = v * 8;
     const int64_t n = byte0 / k_half;
     const int k0 = (int)((byte0 - n * k_half) * 2);
     const int64_t g0 = n * groups + k0 / group_size;
     const v2u w = *reinterpret_cast<const v2u*>(qdata + byte0);
-    const int ng = 16 / group_size;
+    const int ng = group_size >= 16 ? 1 : 16 / group_size;
     float sv[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -68,20 +74,32 @@ __global__ __launch_bounds__(256) void decode_int4_grouped_kernel(
       const uint32_t c = (i & 1) ? (byte >> 4) : (byte & 0xFu);
       const int j = i >> gshift;
       const float s = j == 0 ? sv[0] : (j == 1 ? sv[1] : (j == 2 ? sv[2] : sv[3]));
-      const float p = s_cb[c] * s;  // (tested ahead of the clamp, which would make a NaN of it -127)
-      const int q = p != p ? 0 : (int)fminf(fmaxf(__builtin_rintf(p), -127.0f), 127.0f);
+      const int q = (int)fminf(fmaxf(__builtin_rintf(s_cb[c] * s), -127.0f), 127.0f);
       o[i >> 2] |= (uint32_t)(q & 0xFF) << (8 * (i & 3));
+    }
+    // A NaN product is 0 (the clamp has made it -127); it needs a scale or a level that is not finite.
+    bool off = s_nan != 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) off |= !(fabsf(sv[j]) < INFINITY);
+    if (__builtin_amdgcn_ballot_w64(off)) {
+#pragma unroll 1
+      for (int i = 0; i < 16; ++i) {
+        const uint32_t c = (w[i >> 3] >> (4 * (i & 7))) & 0xFu;
+        const int j = i >> gshift;
+        const float p = s_cb[c] * (j == 0 ? sv[0] : (j == 1 ? sv[1] : (j == 2 ? sv[2] : sv[3])));
+        if (p != p) o[i >> 2] &= ~(0xFFu << (8 * (i & 3)));
+      }
     }
     *reinterpret_cast<v4u*>(out + n * (k_half * 2) + k0) = v4u{o[0], o[1], o[2], o[3]};
   }
 }
 
-// Group sizes that are multiples of 16: a wave per row, 16 weights of one group per lane and vector, four
-// vectors' loads ahead of their decode. The group's 16 levels (level_values) come from a table of the 256
-// e4m3 scales that each workgroup forms once, or from registers (fp32 scales). HBM-bound: 21504 x 5376 at
-// group 16 in 31.1 us with e4m3 scales (5.8 TB/s of the 181 MB it moves) and 35.4 with fp32 ones, where
-// forming every weight's value by itself took 63.3 and 47.9.
-template <bool kE4M3>
+// Group sizes that are multiples of 16: a wave per row, or per piece of a row where the rows are too few for the CUs, 16
+// weights of one group per lane and vector, four vectors' loads ahead of their decode. The group's 16 levels
+// (level_values) come from a table of the 256 e4m3 scales that each workgroup forms once, or from registers (fp32
+// scales). HBM-bound: 21504 x 5376 at group 16 in 30.5 us with e4m3 scales (5.9 TB/s of the 181 MB it moves) and 34.9
+// with fp32 ones, where forming every weight's value by itself took 59.4 and 43.8.
+template <bool kE4M3, bool kPieces>
 __global__ __launch_bounds__(256) void decode_levels_kernel(const uint8_t* __restrict__ qdata, const void* __restrict__ s_rel,
                                                             const float* __restrict__ codebook, int8_t* __restrict__ out,
                                                             int64_t N, int vecs, int groups, int group_size, int gshift) {
@@ -92,35 +110,62 @@ __global__ __launch_bounds__(256) void decode_levels_kernel(const uint8_t* __res
     __syncthreads();
   }
   const int lane = threadIdx.x & 63;
-  for (int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); row < N; row += (int64_t)gridDim.x * 4) {
+  auto decode = [&](int64_t row, int v0) {  // vectors v0 .. v0 + 255 of a row
     const uint8_t* src = qdata + row * vecs * 8;
     int8_t* dst = out + row * vecs * 16;
-    for (int v0 = 0; v0 < vecs; v0 += 4 * kWave) {
-      v2u w[4];
-      uint32_t s[4];
+    v2u w[4];
+    uint32_t s[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int v = min(v0 + j * kWave + lane, vecs - 1);
-        w[j] = __builtin_nontemporal_load(reinterpret_cast<const v2u*>(src + (int64_t)v * 8));
-        const int64_t g = row * groups + (gshift >= 0 ? v * 16 >> gshift : v * 16 / group_size);
-        s[j] = kE4M3 ? reinterpret_cast<const uint8_t*>(s_rel)[g] : reinterpret_cast<const uint32_t*>(s_rel)[g];
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int v = v0 + j * kWave + lane;
-        if (v0 + j * kWave >= vecs) break;
-        v4u t;
-        if constexpr (kE4M3)
-          t = table[s[j]];
-        else
-          t = level_values(levels, __uint_as_float(s[j]));
-        uint32_t o[4];
-        decode8(w[j][0], t, o[0], o[1]);
-        decode8(w[j][1], t, o[2], o[3]);
-        if (v < vecs) *reinterpret_cast<v4u*>(dst + (int64_t)v * 16) = v4u{o[0], o[1], o[2], o[3]};
-      }
+    for (int j = 0; j < 4; ++j) {
+      const int v = min(v0 + j * kWave + lane, vecs - 1);
+      w[j] = __builtin_nontemporal_load(reinterpret_cast<const v2u*>(src + (int64_t)v * 8));
+      const int64_t g = row * groups + (gshift >= 0 ? v * 16 >> gshift : v * 16 / group_size);
+      s[j] = kE4M3 ? reinterpret_cast<const uint8_t*>(s_rel)[g] : reinterpret_cast<const uint32_t*>(s_rel)[g];
     }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int v = v0 + j * kWave + lane;
+      if (v0 + j * kWave >= vecs) break;
+      v4u t;
+      if constexpr (kE4M3)
+        t = table[s[j]];
+      else
+        t = level_values(levels, __uint_as_float(s[j]));
+      uint32_t o[4];
+      decode8(w[j][0], t, o[0], o[1]);
+      decode8(w[j][1], t, o[2], o[3]);
+      if (v < vecs) *reinterpret_cast<v4u*>(dst + (int64_t)v * 16) = v4u{o[0], o[1], o[2], o[3]};
+    }
+  };
+  const int64_t first = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), step = (int64_t)gridDim.x * 4;
+  if constexpr (kPieces) {
+    const int pieces = (vecs + 4 * kWave - 1) / (4 * kWave);
+    for (int64_t i = first; i < N * pieces; i += step) {
+      const int64_t row = i / pieces;
+      decode(row, (int)(i - row * pieces) * (4 * kWave));
+    }
+  } else {
+    for (int64_t row = first; row < N; row += step)
+      for (int v0 = 0; v0 < vecs; v0 += 4 * kWave) decode(row, v0);
   }
+}
+
+// By levels where that was the faster (us per weight, then by levels). e4m3 scales: 1638 x 2048 4.2 and 3.7, 700 x 4096 3.9
+// and 3.8, 700 x 5376 4.2 and 4.7, 1638 x 5376 7.3 and 5.7, 5200 x 784 4.3 and 4.9, 21504 x 1040 13.8 and 11.4. fp32
+// scales, 16 products per vector: 64 x 512 2.6 and 2.4, 700 x 5376 3.6 and 5.2, 2800 x 2048 4.7 and 4.3, 5200 x 1536 5.5
+// and 5.9, 700 x 20480 8.0 and 7.7, 21504 x 1040 11.3 and 13.5.
+static bool decode_by_levels(int64_t N, int64_t K, bool e4m3) {
+  const int64_t weights = N * K, million = 1 << 20;
+  if (e4m3)
+    return (K <= 2048 && N < 2048) ||
+           (K >= 768 && weights >= (K < 1024 ? 8 * million : K <= 4096 ? 5 * million / 2 : 4 * million));
+  return (K < 1024 && N < 1024) || (K >= 2048 && K <= 4096 && weights >= 5 * million) || (K >= 1536 && weights >= 10 * million);
+}
+
+// A wave takes whole rows where there are enough of them, or where a row is one piece (us in rows and in pieces: 4096 x 5376
+// 8.9 and 9.8, 2800 x 5376 7.7 and 8.2, 2800 x 20480 18.4 and 16.7, 1638 x 20480 15.1 and 11.3, 64 x 65536 20.8 and 4.2).
+static bool decode_whole_rows(int64_t N, int64_t K) {
+  return K <= 16 * 4 * kWave || N >= (K < 8192 ? 2048 : 4096);
 }
 
 static int decode_launch(const int8_t* qdata, const void* s_rel, int s_rel_dtype,
@@ -130,19 +175,26 @@ static int decode_launch(const int8_t* qdata, const void* s_rel, int s_rel_dtype
   int64_t blocks = (total_vec + 255) / 256;
   if (blocks > 65536) blocks = 65536;
   if (total_vec == 0) return MXQ_OK;
-  if (group_size % 16 == 0) {
-    const unsigned grid = (unsigned)std::min<int64_t>((N + 3) / 4, 8 * 256);
+  const bool e4m3 = s_rel_dtype == MXQ_DTYPE_E4M3;
+  if (group_size % 16 == 0 && decode_by_levels(N, K, e4m3)) {
     const int shift = (group_size & (group_size - 1)) == 0 ? __builtin_ctzll((unsigned long long)group_size) : -1;
-    if (s_rel_dtype == MXQ_DTYPE_E4M3)
-      decode_levels_kernel<true><<<grid, 256, 0, st>>>((const uint8_t*)qdata, s_rel, codebook, out, N, (int)(K / 16),
-                                                       (int)groups, (int)group_size, shift);
+    const int vecs = (int)(K / 16), g = (int)groups, size = (int)group_size;
+    const int64_t pieces = (vecs + 4 * kWave - 1) / (4 * kWave);
+    const bool rows = decode_whole_rows(N, K);
+    const unsigned grid = (unsigned)std::min<int64_t>(((rows ? N : N * pieces) + 3) / 4, 8 * 256);
+    const uint8_t* q = (const uint8_t*)qdata;
+    if (e4m3 && rows)
+      decode_levels_kernel<true, false><<<grid, 256, 0, st>>>(q, s_rel, codebook, out, N, vecs, g, size, shift);
+    else if (e4m3)
+      decode_levels_kernel<true, true><<<grid, 256, 0, st>>>(q, s_rel, codebook, out, N, vecs, g, size, shift);
+    else if (rows)
+      decode_levels_kernel<false, false><<<grid, 256, 0, st>>>(q, s_rel, codebook, out, N, vecs, g, size, shift);
     else
-      decode_levels_kernel<false><<<grid, 256, 0, st>>>((const uint8_t*)qdata, s_rel, codebook, out, N, (int)(K / 16),
-                                                        (int)groups, (int)group_size, shift);
+      decode_levels_kernel<false, true><<<grid, 256, 0, st>>>(q, s_rel, codebook, out, N, vecs, g, size, shift);
     return mxq_check_launch("decode_levels_kernel");
   }
-  const int gshift = group_size == 4 ? 2 : 3;  // G = 4 or 8
-  if (s_rel_dtype == MXQ_DTYPE_E4M3)
+  const int gshift = group_size == 4 ? 2 : group_size == 8 ? 3 : 4;
+  if (e4m3)
     decode_int4_grouped_kernel<true><<<(unsigned)blocks, 256, 0, st>>>(
         (const uint8_t*)qdata, s_rel, codebook, out, total_vec, k_half, groups, (int)group_size, gshift);
   else
