@@ -72,11 +72,13 @@ def test_quant_fp16_fp32_match_eager(dev, dtype):
     assert torch.equal(s.cpu(), s_ref)
 
 
-# Row widths around the register kernel's edges: one 16-byte chunk, a partly filled wave, a row per
-# wave (3072, 4104) and per workgroup (wide rows and few rows), and widths whose chunks are not aligned.
+# Row widths around the register kernel's edges: too narrow for it (8, 64, many rows of 128), a partly filled wave, a row
+# per wave (up to 1024 columns, 1160 from 2000 rows on, 3072, 4104) and per workgroup (wide rows and few rows), and
+# widths whose chunks are not aligned.
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("m,k", [(1, 8), (3, 520), (5, 2052), (4097, 72), (4100, 3072), (4099, 4104), (7, 14336),
-                                 (4098, 8200), (2, 65536), (9, 1001)])
+                                 (4098, 8200), (2, 65536), (9, 1001), (70, 64), (9, 72), (11, 128), (4100, 128),
+                                 (9, 1024), (1999, 1160), (2001, 1160)])
 def test_quant_row_widths_match_eager(dev, dtype, m, k):
     print(f"quant {dtype} m={m} k={k}", flush=True)
     x = (torch.randn(m, k, generator=gen(m * 7 + k)) * 3).to(dtype)

@@ -42,9 +42,21 @@ MXQ_DEVICE uint32_t gelu_pair(uint32_t w) {
 // least 2^-23 (relative) from a float16 midpoint or is one exactly; in that case it is an fp32 number
 // and q1 equals it. So f16(q1) == f16(x / s) for finite rows; rows with an infinity or NaN divide.
 constexpr int kVecWaves = 4;  // waves of a workgroup: one row each, or one row together
-// One row per wave from this many rows on (both forms take 2310 x 5120 in 9.4-9.7 us; with fewer
-// rows waves run out before the CUs do), if the row fits 16 chunks a lane.
-constexpr int64_t kVecWaveRows = 4096;
+// One row per wave, if the row fits 16 chunks a lane: from 4096 rows on (both forms take 2310 x 5120 in 9.4-9.7 us; with
+// fewer rows waves run out before the CUs do), from 2000 for rows of up to 4 chunks a lane, and always for rows of up to 2,
+// whose workgroup would have little to share (us with a workgroup and a wave per row: bfloat16 4095 x 256 4.5 and
+// 2.9, 1000 x 1024 2.9 and 2.5, 4095 x 1152 5.5 and 3.9, 300 x 1152 2.6 and 2.7). The GELU, a table lookup per value, leaves
+// a wave alone with more work (float16 50 x 1024 2.6 and 3.3, 1000 x 1024 4.1 and 3.6, 2000 x 2048 7.8 and 8.1).
+static bool vec_wave_rows(int64_t rows, int64_t lane_chunks, bool gelu) {
+  if (lane_chunks > 16) return false;
+  return rows >= 4096 || (rows >= (gelu ? 3000 : 2000) && lane_chunks <= 4) || lane_chunks <= (gelu && rows < 512 ? 1 : 2);
+}
+// Rows of so few columns that most lanes of the register kernel's wave have none, while the generic kernel's hold a
+// column each (us, register and generic kernel: float16 60000 x 64 17.8 and 10.1, 60000 x 128 18.1 and 13.7, 1000 x 128 2.2 and 2.3;
+// float32 8000 x 128 3.7 and 3.3; bfloat16 60000 x 64 11.9 and 9.8, 60000 x 128 12.4 and 13.2).
+static bool vec_too_narrow(int x_dtype, int64_t rows, int64_t cols) {
+  return cols <= 64 || (cols <= 128 && rows >= 4000 && x_dtype != MXQ_DTYPE_BF16);
+}
 
 template <int kDtype, int NCH, int kWaves, bool kGelu>
 __global__ __launch_bounds__(kQuantBlock) void quant_rows_vec(const void* __restrict__ xv, int8_t* __restrict__ q,
@@ -814,17 +826,19 @@ extern "C" int mxq_quantize_int8_rowwise_gelu(const void* y_bf16, void* h_bf16, 
   return gelu_wide_launch(y_bf16, h_bf16, q, scales, rows, cols, (hipStream_t)stream);
 }
 
-// The register kernel; false where its alignment or row width does not hold.
+// The register kernel; false where its alignment or row width does not hold, or the generic kernel is faster.
 template <int kDtype, bool kGelu>
 static bool quant_vec_launch_t(const void* x, int8_t* q, float* scales, int64_t rows, int64_t cols, hipStream_t st) {
   constexpr int kPer = kDtype == MXQ_DTYPE_F32 ? 4 : 8;
   if (cols % kPer || (uintptr_t)x % 16 || (uintptr_t)q % kPer || cols > 32 * kPer * kQuantBlock) return false;
+  if (vec_too_narrow(kDtype, rows, cols)) return false;
   const int64_t chunks = cols / kPer;
   const int64_t lane1 = (chunks + kWave - 1) / kWave, lane4 = (chunks + kQuantBlock - 1) / kQuantBlock;
-  if (rows >= kVecWaveRows && lane1 <= 16) {
+  if (vec_wave_rows(rows, lane1, kGelu)) {
     const unsigned grid = row_grid(rows);
 #define MXQ_VEC1(N_) quant_rows_vec<kDtype, N_, 1, kGelu><<<grid, kQuantBlock, 0, st>>>(x, q, scales, rows, (int)cols)
-    if (lane1 <= 2) MXQ_VEC1(2);
+    if (lane1 <= 1) MXQ_VEC1(1);
+    else if (lane1 <= 2) MXQ_VEC1(2);
     else if (lane1 <= 4) MXQ_VEC1(4);
     else if (lane1 <= 8) MXQ_VEC1(8);
     else if (lane1 <= 12) MXQ_VEC1(12);
