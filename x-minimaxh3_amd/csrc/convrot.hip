@@ -590,14 +590,14 @@ UnitSplit unit_split(int units) {
 // than eight waves per CU (156 KB of transpose buffers), two of five to eight, sixteen waves in smaller ones. The
 // throughput split takes over where it has as few units per group (it shares blocks of idle groups between rows: us a row per
 // block and shared, 4096 x 256 6.1 and 3.9, 1300 x 1280 5.7 and 4.5, 1300 x 2560 8.9 and 6.8), and rows of several waves with
-// two units and more per group are not worth a tenth of the groups idle (2048 x 3072 10.1 and 9.3).
+// two units and more per group are not worth an eighth of the unit slots idle (2048 x 3072 10.1 and 9.3).
 UnitSplit few_row_split(int units, int64_t rows, bool mod) {
   const UnitSplit shared = unit_split(units);
   for (int nu = 1; nu <= 4 && (nu < shared.nu || !shared.nu); ++nu) {
     const int gr = (units + nu - 1) / nu, waves = (gr + 3) / 4;
     if (waves > (mod ? 8 : kUnitRowWaves) || (waves > kUnitMaxWaves && nu > 2)) continue;
     // the share of unit slots in use, here units / (4 nu waves)
-    if (nu > 1 && waves > 1 && 10 * shared.waves * shared.nu < 9 * shared.rpb * nu * waves) continue;
+    if (nu > 1 && waves > 1 && 8 * shared.waves * shared.nu < 7 * shared.rpb * nu * waves) continue;
     const int per_cu = waves > 8 ? 1 : waves > kUnitMaxWaves ? 2 : 16 / waves;
     if (rows <= (int64_t)std::min(mxq_cu_count(), 256) * per_cu) return UnitSplit{nu, gr, 1, waves};
   }
