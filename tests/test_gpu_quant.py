@@ -303,10 +303,13 @@ def test_adaln_modulation_groups(dev, m, rows_per_group, d):
 
 # Scale and shift rows over groups of their own: runs of whole rows (equal, nested either way, one
 # of them shared by all), groups that do not nest (read per row), more than 1024 runs of fewer and
-# of at least 4 rows, and rows left over in the last run's wave slots.
+# of at least 4 rows (of wide rows, 1025 by runs and 1501 per row unless one of them is shared by all), four rows in
+# all, and rows left over in the last run's wave slots.
 @pytest.mark.parametrize("m,scale_rows,shift_rows,d", [(35, 7, 7, 5120), (36, 12, 4, 520), (36, 4, 12, 1024),
                                                        (36, 36, 6, 3072), (36, 6, 36, 3072), (36, 9, 6, 512),
-                                                       (2052, 2, 2, 512), (4104, 4, 4, 512)])
+                                                       (2052, 2, 2, 512), (4104, 4, 4, 512), (4, 2, 2, 1536),
+                                                       (4100, 4, 4, 5376), (6004, 4, 4, 4608),
+                                                       (6010, 6010, 5, 4608)])
 def test_adaln_quant_runs(dev, m, scale_rows, shift_rows, d):
     x = activations(m, d, 78)
     sc = (torch.randn(m // scale_rows, d, generator=gen(1)) * 0.1).to(torch.bfloat16)

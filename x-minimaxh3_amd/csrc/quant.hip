@@ -492,6 +492,17 @@ constexpr int kAdalnRows = 16;
 // 235, of 2 and 1 rows 294 and 699 against 237 and 271 (3072 columns: 161 and 275 against 289 and 292);
 // 960 rows in runs of 1 row 15.0 against 38.5.
 constexpr int64_t kAdalnMinRun = 4, kAdalnFewRuns = 1024;
+// Widths of 4104 to 6144 columns but for 5120 leave a SIMD two waves of that kernel, so that many short runs are better
+// off per row if both modulations change with them (us per row and by runs, 5376 columns: 1025 runs of 4 rows 56 and
+// 38, 2000 of 4 69 and 81, 2000 of 5 116 and 101, 7000 of 5 299 and 327, 7000 of 6 no difference). So are four rows
+// and fewer of widths that are not the kernel's own (4 x 4608 in 2 runs 8.5 and 9.3, 4 x 3072 7.9 and 6.4).
+static bool adaln_by_runs(int64_t rows, int64_t run, int64_t runs, int64_t cols, int chunks, bool both) {
+  const bool light = cols == chunks * 512 && chunks <= 10;  // whole lanes, three waves a SIMD
+  if (runs == 1) return true;
+  if (rows <= 4 && !light) return false;
+  if (both && !light && cols > 4096 && cols <= 6144 && run >= kAdalnMinRun && run < 6) return runs <= (run < 5 ? 1500 : 4000);
+  return runs <= kAdalnFewRuns || (run >= kAdalnMinRun && runs <= 65535);
+}
 constexpr int kAdalnMaxCols = 8192;
 
 template <int NCH, bool kQuant>
@@ -973,7 +984,7 @@ static int adaln_launch(const void* x, const void* scale, const void* shift, int
   else if (shift_group >= rows || shift_group % scale_group == 0)
     run = scale_group;
   const int64_t runs = run ? (rows + run - 1) / run : 0;
-  if (run && (runs <= kAdalnFewRuns || (run >= kAdalnMinRun && runs <= 65535)) && cols <= kAdalnMaxCols && (cols == uch * 512 || uch <= 12)) {
+  if (run && adaln_by_runs(rows, run, runs, cols, uch, scale_group < rows && shift_group < rows) && cols <= kAdalnMaxCols && (cols == uch * 512 || uch <= 12)) {
     // few modulation rows: the two-buffer kernel (widths whose register budget it fits)
     // Every workgroup takes an equal share of the rows, so the grid is what fits on the device at
     // once: a larger one left its last workgroups to start after the first had finished.
