@@ -1556,9 +1556,11 @@ constexpr TileCost kTileCostShortK = {{100, 685}, {92, 705}, {62, 955}, {64, 555
 constexpr int64_t kShortK = 4096;
 // Gated residual: the epilogue also reads and writes the residual, and large tiles do that all at once, with no other
 // workgroup's products beside it (4331 x 3072 x 3072 in 256-row tiles, as the costs above have it, 125 us, in 128 x 128
-// ones 90). Fitted to 420 shapes of K = 2048 to 20480: 5.6 % above the fastest on average with the costs above, 4.8 % with
-// these, and 2 % and more slower than the uniform plan in 7 of them, where it was 75.
+// ones 90); with more than a round of 256-row tiles the next tile's loads run beside it. Fitted to 208 shapes of up to a round,
+// 4.1 % above the fastest on average and 2 % and more slower than the uniform plan in 2 (5.6 % and 34 with the costs
+// above), and 212 of more, 4.2 % and 12 (5.7 % and 41).
 constexpr TileCost kTileCostGated = {{100, 1680}, {77, 1390}, {56, 770}, {60, 120}, {37, 380}};
+constexpr TileCost kTileCostGatedRounds = {{100, 775}, {88, 755}, {65, 565}, {61, 645}, {36, 10}};
 struct ShortPlan {
   int rows;        // rows of a short tile: 192 or 128; 256: whole 256-tiles in place of 128-tiles; 0: plan_gemm's
   int tiles_m;     // 256-row tile-rows
@@ -1589,7 +1591,9 @@ static ShortPlan short_plan(int64_t M, int64_t N, int64_t K, int table, const Ge
   const int64_t cus = std::max(1, mxq_cu_count()), tm = (M + 255) / 256, tn = (N + 255) / 256;
   if (table == kTableGelu || g.deep || K < 2048 || tm > 6 * cus || tm * tn > 6 * cus) return best;
   const bool counters = workspace_bytes >= kShortQueueBytes;
-  const TileCost& cost = table == kGatedResidual ? kTileCostGated : K < kShortK ? kTileCostShortK : kTileCost;
+  const TileCost& cost = table == kGatedResidual ? (tm * tn > cus ? kTileCostGatedRounds : kTileCostGated)
+                         : K < kShortK           ? kTileCostShortK
+                                                 : kTileCost;
   const int64_t c256 = cost.t256.at(K), whole = tile_span(tm * tn, c256, 0, 0, cus);
   int64_t least = whole;
   if (g.tile == 128) {
