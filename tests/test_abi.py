@@ -429,7 +429,7 @@ def test_gemm_workspace_is_asked_for_on_the_launch_device(monkeypatch):
 
     @contextlib.contextmanager
     def device(d):
-        before, current[0] = current[0], torch.device(d).index
+        before, current[0] = current[0], d if isinstance(d, int) else d.index
         yield
         current[0] = before
 
@@ -444,14 +444,14 @@ def test_gemm_workspace_is_asked_for_on_the_launch_device(monkeypatch):
     monkeypatch.setattr(ops, "_raw_stream", lambda index: 7)
     kept = torch.zeros(_lib.GEMM_WORKSPACE_BYTES, dtype=torch.uint8)
     monkeypatch.setattr(ops, "_GEMM_WORKSPACES", {(0, 7): kept})
-    _lib.gemm_workspace_bytes.cache_clear()
+    ops._workspace_bytes.cache_clear()
     try:
         for _ in range(2):  # asked, then kept
             assert ops._gemm_ws(torch.device("cuda:0"), 4097, 21504, 5376)[1] == _lib.GEMM_WORKSPACE_BYTES
             assert ops._gemm_ws(torch.device("cuda:1"), 4097, 21504, 5376) == (None, 0)
         assert asked == [0, 1] and current[0] == 0
     finally:
-        _lib.gemm_workspace_bytes.cache_clear()
+        ops._workspace_bytes.cache_clear()
 
 
 @pytest.mark.parametrize("other", [dict(mxq_of_a_later_version=[]), 99])

@@ -8,7 +8,6 @@ is raised.
 from __future__ import annotations
 
 import ctypes
-import functools
 import pathlib
 import threading
 
@@ -135,11 +134,10 @@ def gemm_short_plan(m: int, n: int, k: int, table: int = 0, workspace_bytes: int
     return {"rows": out[0], "tiles_m": out[1], "short_m": out[2], "queued": bool(out[3])}
 
 
-@functools.lru_cache(maxsize=4096)
-def gemm_workspace_bytes(m: int, n: int, k: int, table: int = 0, device: int | None = None) -> int:
+def gemm_workspace_bytes(m: int, n: int, k: int, table: int = 0) -> int:
     """Workspace an INT8 GEMM of this shape can use (mxq_int8_gemm_workspace): none, the tile-queue
     counters, or those with room for the partial sums of a K split. The library answers for the current
-    device, whose CUs its plans fill; ``device`` is that device's index, so that answers are kept apart."""
+    device, whose CUs its plans fill."""
     out = ctypes.c_int64()
     call("mxq_int8_gemm_workspace", m, n, k, int(table), ctypes.byref(out))
     return out.value

@@ -10,6 +10,7 @@ on the tensors' GPU and current stream; there is no CPU path.
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 
@@ -35,9 +36,8 @@ def _stream(device: torch.device):
 # only when it is not the current one, and a factor that is already float32 (or the output dtype),
 # contiguous and in place passes through without a chain of no-op conversions. One int8_linear of two
 # launches: 41 -> 20 us of host time (one row 24 -> 16, the row quantizer alone 15 -> 9).
-def _raw_stream(index: int) -> int:
-    # (looked up when called: a CPU build of torch has no such function and still imports this module)
-    return torch._C._cuda_getCurrentRawStream(index)
+# (None in a CPU build of torch, which still imports this module)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _ptr(t: torch.Tensor | None):
@@ -68,6 +68,13 @@ def _vector(t: torch.Tensor, dtype: torch.dtype, dev: torch.device) -> torch.Ten
 _GEMM_WORKSPACES: dict[tuple[int, int], torch.Tensor] = {}
 
 
+@functools.lru_cache(maxsize=4096)
+def _workspace_bytes(m: int, n: int, k: int, table: int, index: int) -> int:
+    """The library's answer for device ``index``, asked with it current; one kept per device."""
+    with torch.cuda.device(index):
+        return _lib.gemm_workspace_bytes(m, n, k, table)
+
+
 def _gemm_ws(device: torch.device, m: int = 0, n: int = 0, k: int = 0, table: int = 0):
     """The workspace of an INT8 GEMM of this shape on ``device``'s current stream, as the two
     trailing arguments (pointer, bytes) the GEMM entry points take before the stream: the
@@ -83,11 +90,8 @@ def _gemm_ws(device: torch.device, m: int = 0, n: int = 0, k: int = 0, table: in
     GEMM_WORKSPACE_BYTES, where other launches keep their counters, are not cleared: a problem that splits
     uses none, nor does a narrower one given the same workspace (a last column chunk). That holds for the plan of
     the device the launch runs on, so the library is asked with that device current."""
-    if torch.cuda.current_device() != device.index:
-        with torch.cuda.device(device):
-            return _gemm_ws(device, m, n, k, table)
     if m:
-        need = _lib.gemm_workspace_bytes(m, n, k, table, device.index)
+        need = _workspace_bytes(m, n, k, table, device.index)
         if need == 0:  # neither a queue nor a split
             return None, 0
         if need > _lib.GEMM_WORKSPACE_BYTES:
@@ -95,7 +99,12 @@ def _gemm_ws(device: torch.device, m: int = 0, n: int = 0, k: int = 0, table: in
             ptr = _p(part)
             ptr.keep = part
             return ptr, need
-    if torch.cuda.is_current_stream_capturing():
+    if torch.cuda.current_device() == device.index:
+        capturing = torch.cuda.is_current_stream_capturing()
+    else:
+        with torch.cuda.device(device):
+            capturing = torch.cuda.is_current_stream_capturing()
+    if capturing:
         return None, 0
     key = (device.index, _raw_stream(device.index))
     ws = _GEMM_WORKSPACES.get(key)
