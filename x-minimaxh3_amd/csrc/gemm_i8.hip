@@ -1472,7 +1472,9 @@ struct GemmPlan {
 // of 128-tiles, and a round of 128-tiles takes about 0.55 of a round of 256-tiles (measured at
 // K = 4096-8192), so a last round of 256-tiles that is mostly empty is cheaper as 128-tiles
 // (4096 x 5120: 1.25 rounds, 0.147 -> 0.117 ms) and a full one is not. The table epilogues (GELU,
-// SwiGLU) need the 256-tile ring. With a workspace, problems of two rounds or more balance their
+// SwiGLU) need the 256-tile ring. (0.55 is low: the fits behind TileCost give 0.60 to 0.70, which decide from K = 2048 up
+// to six rounds; past those it still takes 128-tiles in windows of 128 rows, 3329 x 28672 the first, where 256-tiles
+// end sooner.) With a workspace, problems of two rounds or more balance their
 // tiles over the XCDs at run time (pick_tile).
 static GemmPlan plan_gemm(int64_t M, int64_t N, int table, int64_t workspace_bytes) {
   GemmPlan g{};
